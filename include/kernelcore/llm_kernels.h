@@ -62,8 +62,8 @@ typedef struct kcMatvecQ4Q8Args {
 
 /* matmul_{q4k,q6k}_q8x{4,8} (per-32 slots) and matmul_{q4k,q6k}_q8kx{4,8} (per-256 slots),
  * llm_kernels.hpp:262-271: Y = W X, column c from slot xq + c * slot_ints, written to y + c * rows.
- * On the GPU the x4 / x8 names are the same kernels (a column-tiled kernel, bit-exact per column,
- * and for Q4_K with per-256 slots and >= 32 columns the MFMA kernel); row_block is validated
+ * On the GPU the x4 / x8 names are the same kernels (a column-tiled kernel for per-32 slots, a matrix-core
+ * kernel for per-256 slots, both bit-exact per column, and from 64 per-256 columns the prefill kernel); row_block is validated
  * (> 0) and otherwise unused. */
 typedef struct kcMatmulKQ8Args {
     const int* qw;

@@ -9,12 +9,14 @@
 // computing NC columns from one load of its weights, and the per-row sum of super-block terms
 // done in registers in super-block order (the four lanes of a row pass their terms with
 // cross-lane reads, in order), which keeps every column bit-identical to the reference. It serves
-// small batches and the per-32 names; large per-256 batches go to the MFMA kernel.
+// the per-32 names and single columns; per-256 batches go to the MFMA kernels (kmatmul_short.hip, and
+// from 64 columns the prefill kernels).
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
 
 #include "internal.hpp"
+#include "kmatmul_short.hpp"
 #include "kquant.hpp"
 #include "kquant_device.hpp"
 #include "launch.hpp"
@@ -159,15 +161,23 @@ int launchMatmulCols(bool q6k, bool per256, const kcMatmulKQ8Args& a, hipStream_
     return per256 ? pickCols<false, true>(a, s) : pickCols<false, false>(a, s);
 }
 
+int launchMatmulFew(bool q6k, bool per256, const kcMatmulKQ8Args& a, hipStream_t s) {
+    if (per256 && matmulShortRuns(a.k, a.ncols))
+        return launchMatmulShort(ShortGroup{{{reinterpret_cast<const uint8_t*>(a.qw), a.y, a.rows, q6k, 0}}, 1}, a.xq, a.k,
+                                 a.ncols, s);
+    return launchMatmulCols(q6k, per256, a, s);
+}
+
 int launchMatmulKq(bool q6k, bool per256, const kcMatmulKQ8Args& a, hipStream_t s) {
-    // "matmul_path": 0 default (MFMA from 64 columns with per-256 slots), 1 column tiles; 2 and up
+    // "matmul_path": 0 default (per-256 slots: the short-batch kernel, the
+    // prefill MFMA kernel from 64 columns), 1 column tiles; 2 and up
     // force the MFMA kernels: 2 default MFMA kernel, 3 register-staged 2 x 2 blocks per wavefront,
     // 4 / 5 register-staged one-wavefront-per-SIMD rows (two / one super-block groups), 7 the
     // wide-tile kernel (kmatmul_mfmaw.hip).
     const int path = option("matmul_path");
     const bool mfma = per256 && (path >= 2 || (path == 0 && a.ncols >= 64));
     if (mfma) return launchMatmulMfma(q6k, a, s);
-    return launchMatmulCols(q6k, per256, a, s);
+    return launchMatmulFew(q6k, per256, a, s);
 }
 
 }  // namespace kcamd

@@ -44,6 +44,7 @@
 #include "internal.hpp"
 #include "kquant.hpp"
 #include "kmatmul_mfma.hpp"
+#include "kmatmul_short.hpp"
 #include "launch.hpp"
 
 namespace kcamd {
@@ -1274,7 +1275,7 @@ size_t fixedScratchBytes() { return kFixedScratchBytes; }
 int launchMatmulKqNoAlloc(bool q6k, bool per256, const kcMatmulKQ8Args& a, hipStream_t s) {
     const int path = option("matmul_path");
     const bool mfma = per256 && (path >= 2 || (path == 0 && a.ncols >= 64));
-    if (!mfma) return launchMatmulCols(q6k, per256, a, s);  // the column kernel stages nothing
+    if (!mfma) return launchMatmulFew(q6k, per256, a, s);  // (these kernels stage nothing)
     if (path == 3) return q6k ? runMfma<true>(a, s) : runMfma<false>(a, s);
     if (path == 4) return q6k ? runMfma8<true, 2>(a, s) : runMfma8<false, 2>(a, s);
     if (path == 5) return q6k ? runMfma8<true, 1>(a, s) : runMfma8<false, 1>(a, s);
@@ -1366,6 +1367,13 @@ int launchMatmulGroup(const MmPart* parts, int nparts, const int* xq, int k, int
             *used_ks = ks;
             return runMfmaH(parts, nparts, xq, k, ncols, ks, act, s, nullptr, part_ks);
         }
+    }
+    if (option("matmul_path") == 0 && matmulShortRuns(k, ncols)) {  // one launch for the group
+        ShortGroup g{};
+        g.nparts = nparts;
+        for (int i = 0; i < nparts; ++i)
+            g.p[i] = ShortPart{static_cast<const uint8_t*>(parts[i].qw), parts[i].y[0], parts[i].rows, parts[i].q6, 0};
+        return launchMatmulShort(g, xq, k, ncols, s);
     }
     for (int i = 0; i < nparts; ++i) {  // one matmul per part, no K split
         const kcMatmulKQ8Args a{static_cast<const int*>(parts[i].qw), xq, parts[i].y[0], nullptr, parts[i].rows, k,

@@ -39,6 +39,9 @@ int launchQuantizeColsK(const float* x, int* q, int k, int ncols, hipStream_t s,
 int launchMatvecKq(bool q6k, const kcMatvecQ4Q8Args& a, hipStream_t s);
 // kmatmul.hip: column-tiled matmul (any ncols; bit-identical per column to the reference).
 int launchMatmulCols(bool q6k, bool per256, const kcMatmulKQ8Args& a, hipStream_t s);
+// The batches the prefill MFMA kernel does not take: per-256 slots on the short-batch kernel
+// (kmatmul_short.hip), else column tiles.
+int launchMatmulFew(bool q6k, bool per256, const kcMatmulKQ8Args& a, hipStream_t s);
 // kmatmul_mfma.hip: K-quant x per-256 activations on MFMA (large batches).
 int launchMatmulMfma(bool q6k, const kcMatmulKQ8Args& a, hipStream_t s);
 // The per-stream scratch a by-name per-256 matmul of these sizes stages its fp16 activations (and

@@ -1,0 +1,42 @@
+"""The short-batch per-256 matmul (kmatmul_short.hip) at the edges of its tiles: 1 to 4 blocks of 16 columns,
+ragged columns and rows, slot rows that are not 16-byte aligned (k / 256 not a multiple of 4, and slots at an
+odd word), rounds of super-blocks (long rows), both wavefront counts. Integer sums and the reference's float
+operations in its order: bit-exact against the oracle."""
+import numpy as np
+import pytest
+
+import kernelcore_amd as kc
+import oracle
+from tests import kq
+from tests.test_gpu_matmul import oracle_slots
+
+pytestmark = pytest.mark.gpu
+O = oracle.lib()
+
+
+@pytest.fixture(scope="module", autouse=True)
+def runtime():
+    kc.init()
+    yield
+    kc.synchronize()
+
+
+@pytest.mark.parametrize("qtype", ["q4k", "q6k"])
+@pytest.mark.parametrize("rows,k,ncols,shift", [
+    (8, 256, 2, 0), (24, 1024, 16, 0), (40, 1024, 17, 0), (200, 1280, 33, 0), (1000, 2048, 63, 0), (16, 4096, 15, 0),
+    (136, 12288, 40, 0), (24, 16384, 50, 0), (72, 8192, 62, 0), (48, 1024, 31, 1),
+])
+def test_short_batch_is_bit_exact(qtype, rows, k, ncols, shift):
+    print(f"short batch {qtype} {rows}x{k} ncols={ncols} shift={shift}", flush=True)
+    w = kq.random_blocks(qtype, rows, k, seed=rows + k + ncols)
+    x = kq.randn(k * ncols, ncols + rows, 1.5)
+    q = oracle_slots(x, k, ncols, True)
+    stream, y = kc.upload_weights(qtype, w, rows, k), kc.Buffer(4 * rows * ncols)
+    at = kc.Buffer(q.nbytes + 4 * shift)
+    at.upload(q, 4 * shift)
+    kc.launch(f"matmul_{qtype}_q8kx8", kc.MatmulKQ8Args(stream.ptr, at.at(4 * shift), y.ptr, None, rows, k, ncols, 8))
+    want = np.zeros(rows * ncols, np.float32)
+    getattr(O, f"kco_matmul_{qtype}_q8k")(w, q, want, rows, k, ncols)
+    assert np.array_equal(kq.bits(y.download(np.float32)), kq.bits(want))
+    for b in (stream, at, y):
+        b.free()
