@@ -10,7 +10,7 @@
 //   * ncols <= 8 (decode): one wavefront per 2 rows; each lane multiplies 8 consecutive values of
 //     a row with the same 8 values of every column, the partial sums are reduced across the 64
 //     lanes. HBM-bound (2 bytes per weight).
-//   * ncols > 8: v_mfma_f32_32x32x16_f16 on 32 x 32 output tiles, four per workgroup. The weights
+//   * ncols > 8: v_mfma_f32_16x16x32_f16, K split over the wavefronts of a workgroup. The weights
 //     are exact fp16 operands; each activation is split into hi = fp16(x) and lo = fp16(x - hi)
 //     and every product runs as two MFMAs (f32 accumulation), within about 2^-22 of the fp32
 //     product (a single fp16 rounding of x would be 2^-11).
@@ -29,7 +29,8 @@ namespace kcamd {
 namespace {
 
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ float h2f(uint32_t bits) { return (float)__builtin_bit_cast(_Float16, (uint16_t)bits); }
@@ -96,69 +97,146 @@ __global__ __launch_bounds__(256) void mmf16_vec_kernel(const uint16_t* __restri
         }
 }
 
-// ---- ncols > 8, k % 16 == 0: a workgroup of 4 wavefronts covers 64 rows x 64 columns, each
-// wavefront one 32 x 32 tile. Lane (j, h) (j = lane % 32, h = lane / 32) holds, per K-step of 16,
-// A = W[row0 + j][k0 + 8h .. +8] and B = x[col0 + j][k0 + 8h .. +8]; the accumulator's register
-// v holds output row 8 (v / 4) + 4 h + v % 4 of column j. Rows and columns past the end reread
-// the last ones and are not stored.
-__global__ __launch_bounds__(256) void mmf16_mfma_kernel(const uint16_t* __restrict__ w, const float* __restrict__ x,
-                                                         float* __restrict__ y, int rows, int k, int ncols) {
-    constexpr int U = 4;  // K-steps whose loads are issued together
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, j = lane & 31, h = lane >> 5;
-    const int row0 = blockIdx.x * 64 + (wave & 1) * 32, col0 = blockIdx.y * 64 + (wave >> 1) * 32;
-    if (row0 >= rows || col0 >= ncols) return;
-    const uint16_t* wr = w + (size_t)min(row0 + j, rows - 1) * k + 8 * h;
-    const float* xr = x + (size_t)min(col0 + j, ncols - 1) * k + 8 * h;
-    f32x16 acc = {};
-    const int steps = k / 16;
-    int st = 0;
-    for (; st + U <= steps; st += U) {
-        h8 a[U];
-        float4 xv[U][2];
+// ---- ncols > 8, k % 16 == 0: a workgroup of 8 wavefronts covers 16 T rows x 16 C columns; K advances in
+// chunks of 256 values, wavefront w taking values 32 w .. 32 w + 31 of each (one v_mfma_f32_16x16x32_f16 per 16 x 16
+// block and activation part), and the 8 partial sums meet in LDS at the end. Lane (r = lane % 16, kg = lane / 16)
+// holds A = W[row0 + 16 t + r][k + 8 kg .. +8] and B = x[col0 + 16 c + r][k + 8 kg .. +8]; the result's register e is
+// row 4 kg + e of column r. Rows and columns past the end reread the last ones and are not stored.
+//
+// The chunks come by buffer-to-LDS loads of whole row pieces (512 B of a weight row, 1 KiB of a column), S stages
+// deep: operand loads straight from memory touch 16 rows' cache lines per instruction, about 54 cycles each,
+// and that bound the kernel (1024 x 4096, 77 columns: 16.5 us so, 10 us from LDS; 101 us for one wavefront per
+// 32 x 32 block over all of K). A 16-byte piece p of row or column i lies at chunk
+// p ^ (i % 16), so the 16 rows an operand read touches lie in different banks.
+__device__ __forceinline__ void splitHiLo(const float4& x0, const float4& x1, h8& hi, h8& lo) {
+    const float xs[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            a[u] = __builtin_nontemporal_load(reinterpret_cast<const h8*>(wr + 16 * (st + u)));
-            const float4* xp = reinterpret_cast<const float4*>(xr + 16 * (st + u));
-            xv[u][0] = xp[0];
-            xv[u][1] = xp[1];
+    for (int e = 0; e < 8; ++e) {
+        const _Float16 h = (_Float16)xs[e];
+        hi[e] = h;
+        lo[e] = (_Float16)(xs[e] - (float)h);
+    }
+}
+
+typedef __attribute__((address_space(3))) void* LdsPtr;
+constexpr int kF16Waves = 8;
+template <int T, int C>
+constexpr int f16StageBytes() { return T * 16 * 512 + C * 16 * 1024; }
+
+template <int T, int C, int S>
+__device__ __forceinline__ void f16Tile(float4* lds4, const uint16_t* __restrict__ w, const float* __restrict__ x,
+                                        float* __restrict__ y, int rows, int k, int ncols) {
+    constexpr int kStage = f16StageBytes<T, C>(), kLoads = T + 2 * C;  // loads per wavefront and stage
+    char* lds = reinterpret_cast<char*>(lds4);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, r = lane & 15, kg = lane >> 4;
+    const int row0 = blockIdx.x * 16 * T, col0 = blockIdx.y * 16 * C;
+    const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint16_t*>(w + (size_t)row0 * k), (short)0, (int)((uint32_t)min(16 * T, rows - row0) * (uint32_t)k * 2u), 0x00020000);
+    const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float*>(x + (size_t)col0 * k), (short)0, (int)((uint32_t)min(16 * C, ncols - col0) * (uint32_t)k * 4u), 0x00020000);
+    // this lane's piece of each of its wavefront's loads: weight load 8 i + wave holds rows 2 (8 i + wave), + 1;
+    // column load 8 i + wave that column
+    uint32_t wo[T], xo[2 * C];  // byte offset of the row
+    int wp[T], xp[2 * C];       // piece within the chunk
+#pragma unroll
+    for (int i = 0; i < T; ++i) {
+        const int row = 2 * (8 * i + wave) + (lane >> 5);
+        wo[i] = (uint32_t)min(row, rows - row0 - 1) * (uint32_t)k * 2u;
+        wp[i] = (lane & 31) ^ (row & 15);
+    }
+#pragma unroll
+    for (int i = 0; i < 2 * C; ++i) {
+        const int col = 8 * i + wave;
+        xo[i] = (uint32_t)min(col, ncols - col0 - 1) * (uint32_t)k * 4u;
+        xp[i] = lane ^ (col & 15);
+    }
+    const int nch = (k + 255) / 256;
+    auto stage = [&](int ch) {  // (chunks past the end: the last one again, unused; pieces past k: the row's first)
+        char* buf = lds + (ch % S) * kStage;
+        const int k0 = min(ch, nch - 1) * 256;
+#pragma unroll
+        for (int i = 0; i < T; ++i)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (LdsPtr)(buf + (8 * i + wave) * 1024), 16,
+                                                     wo[i] + (k0 + 8 * wp[i] < k ? (uint32_t)(k0 * 2 + 16 * wp[i]) : 0u), 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 2 * C; ++i)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (LdsPtr)(buf + T * 8192 + (8 * i + wave) * 1024), 16,
+                                                     xo[i] + (k0 + 4 * xp[i] < k ? (uint32_t)(k0 * 4 + 16 * xp[i]) : 0u), 0, 0, 0);
+    };
+    f32x4 acc[T][C] = {}, sum[T][C] = {};
+#pragma unroll
+    for (int i = 0; i < S - 1; ++i) stage(i);
+    const int pw = 4 * wave + kg;  // this lane's weight piece
+    for (int ch = 0; ch < nch; ++ch) {
+        // chunk ch has landed (S - 2 later ones may be in flight), everywhere; chunk ch - 1 has been read
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((S - 2) * kLoads) : "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        stage(ch + S - 1);
+        const char* buf = lds + (ch % S) * kStage;
+        h8 hi[C], lo[C], a[T];
+#pragma unroll
+        for (int t = 0; t < T; ++t) a[t] = *reinterpret_cast<const h8*>(buf + (16 * t + r) * 512 + ((pw ^ r) * 16));
+#pragma unroll
+        for (int c = 0; c < C; ++c) {
+            const char* b = buf + T * 8192 + (16 * c + r) * 1024;
+            splitHiLo(*reinterpret_cast<const float4*>(b + ((2 * pw) ^ r) * 16),
+                      *reinterpret_cast<const float4*>(b + ((2 * pw + 1) ^ r) * 16), hi[c], lo[c]);
         }
+        if (ch == nch - 1 && k % 256) {  // the values past k
+            const bool in = ch * 256 + 8 * pw < k;
+            const h8 zero = {};
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const float xs[8] = {xv[u][0].x, xv[u][0].y, xv[u][0].z, xv[u][0].w,
-                                 xv[u][1].x, xv[u][1].y, xv[u][1].z, xv[u][1].w};
-            h8 bh, bl;
+            for (int t = 0; t < T; ++t) a[t] = in ? a[t] : zero;
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const _Float16 hi = (_Float16)xs[e];
-                bh[e] = hi;
-                bl[e] = (_Float16)(xs[e] - (float)hi);
+            for (int c = 0; c < C; ++c) {
+                hi[c] = in ? hi[c] : zero;
+                lo[c] = in ? lo[c] : zero;
             }
-            acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[u], bh, acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[u], bl, acc, 0, 0, 0);
         }
-    }
-    for (; st < steps; ++st) {
-        const h8 a = *reinterpret_cast<const h8*>(wr + 16 * st);
-        const float4* xp = reinterpret_cast<const float4*>(xr + 16 * st);
-        const float4 x0 = xp[0], x1 = xp[1];
-        const float xs[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
-        h8 bh, bl;
+        // each chunk's products start from zero and are added to the sum while the next chunk's run: the rounding of one
+        // long chain of accumulations was most of the error (2.2e-7 at k = 4096, 1.2e-7 so)
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const _Float16 hi = (_Float16)xs[e];
-            bh[e] = hi;
-            bl[e] = (_Float16)(xs[e] - (float)hi);
+        for (int t = 0; t < T; ++t)
+#pragma unroll
+            for (int c = 0; c < C; ++c) {
+                sum[t][c] += acc[t][c];
+                acc[t][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[t], lo[c], f32x4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+                acc[t][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[t], hi[c], acc[t][c], 0, 0, 0);
+            }
+    }
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");  // (the stages past the end)
+    __syncthreads();
+    float4* part = lds4;  // [wavefront][t][c][lane]
+#pragma unroll
+    for (int t = 0; t < T; ++t)
+#pragma unroll
+        for (int c = 0; c < C; ++c) {
+            sum[t][c] += acc[t][c];
+            part[((wave * T + t) * C + c) * 64 + lane] = make_float4(sum[t][c][0], sum[t][c][1], sum[t][c][2], sum[t][c][3]);
         }
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, bh, acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, bl, acc, 0, 0, 0);
-    }
-    const int col = col0 + j;
-    if (col >= ncols) return;
+    __syncthreads();
+    for (int i = threadIdx.x; i < T * C * 64; i += blockDim.x) {
+        f32x4u o = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-    for (int v = 0; v < 16; ++v) {
-        const int row = row0 + 8 * (v / 4) + 4 * h + (v % 4);
-        if (row < rows) y[(size_t)col * rows + row] = acc[v];
+        for (int v = 0; v < kF16Waves; ++v) {
+            const float4 q = part[v * T * C * 64 + i];
+            o[0] += q.x;
+            o[1] += q.y;
+            o[2] += q.z;
+            o[3] += q.w;
+        }
+        const int l = i & 63, tc = i >> 6, row = row0 + 16 * (tc / C) + 4 * (l >> 4), col = col0 + 16 * (tc % C) + (l & 15);
+        if (row < rows && col < ncols) *reinterpret_cast<f32x4u*>(y + (size_t)col * rows + row) = o;  // rows % 8 == 0
     }
+}
+
+template <int T, int C, int S>
+__global__ __launch_bounds__(64 * kF16Waves) void mmf16_mfma_kernel(const uint16_t* __restrict__ w,
+                                                                    const float* __restrict__ x, float* __restrict__ y,
+                                                                    int rows, int k, int ncols) {
+    extern __shared__ float4 lds4[];
+    f16Tile<T, C, S>(lds4, w, x, y, rows, k, ncols);
 }
 
 // ---- any even k: one thread per (row, column), the reference's loop (llm_reference.cpp:756-764).
@@ -197,9 +275,29 @@ int launchMatmulF16(const void* w, const float* x, float* y, int rows, int k, in
             else if (nc <= 4) hipLaunchKernelGGL(mmf16_vec_kernel<4>, grid, block, 0, s, wh, xc, yc, rows, k, nc);
             else hipLaunchKernelGGL(mmf16_vec_kernel<8>, grid, block, 0, s, wh, xc, yc, rows, k, nc);
         }
-    } else if (a16 && k % 16 == 0) {
-        const dim3 grid((rows + 63) / 64, (ncols + 63) / 64), block(256);
-        hipLaunchKernelGGL(mmf16_mfma_kernel, grid, block, 0, s, wh, x, y, rows, k, ncols);
+    } else if (a16 && k % 16 == 0 && (unsigned long long)k * 128 < (1ull << 32) && ncols <= 1 << 20) {
+        // (a tile's 32-bit byte offsets, the grid's second dimension)
+        // the smallest tile whose workgroups run at once on the 256 CUs (a second round costs more than a larger
+        // tile: 1024 x 4096, 77 columns 12.4 us on 16 x 16 (320 workgroups), 9.9 us on 32 x 16 (160), 11.3 us on
+        // 64 x 16 (80)), else the largest (512 columns: 18.7 us on 64 x 32, 22.5 us on 64 x 16); three stages where they
+        // fit
+        const auto wgs = [&](int t, int c) { return (long long)((rows + 16 * t - 1) / (16 * t)) * ((ncols + 16 * c - 1) / (16 * c)); };
+        const dim3 block(64 * kF16Waves);
+#define KC_F16(TT, CC, SS)                                                                                             \
+    {                                                                                                                  \
+        constexpr int lds = SS * f16StageBytes<TT, CC>();                                                              \
+        static_assert(lds >= kF16Waves * TT * CC * 1024, "the partial sums reuse the stages");                         \
+        static const int attr = (int)hipFuncSetAttribute(reinterpret_cast<const void*>(mmf16_mfma_kernel<TT, CC, SS>), \
+                                                         hipFuncAttributeMaxDynamicSharedMemorySize, lds);             \
+        if (attr != 0) return fromHip(attr, "matmul_f16: LDS size");                                                   \
+        hipLaunchKernelGGL((mmf16_mfma_kernel<TT, CC, SS>), dim3((rows + 16 * TT - 1) / (16 * TT),                     \
+                           (ncols + 16 * CC - 1) / (16 * CC)), block, lds, s, wh, x, y, rows, k, ncols);               \
+    }
+        if (wgs(1, 1) <= 256) KC_F16(1, 1, 3)
+        else if (wgs(2, 1) <= 256) KC_F16(2, 1, 3)
+        else if (wgs(4, 1) <= 256) KC_F16(4, 1, 3)
+        else KC_F16(4, 2, 2)
+#undef KC_F16
     } else {
         const long long n = (long long)rows * ncols;
         hipLaunchKernelGGL(mmf16_simple_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s,
