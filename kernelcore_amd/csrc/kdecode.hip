@@ -1225,6 +1225,20 @@ __global__ __launch_bounds__(256) void flash_decode_kernel(const float* __restri
     }
 }
 
+// The head's D outputs in LDS quantized per 32 into the token's per-32 slot (eight lanes per block, four values
+// each).
+template <int D>
+__device__ __forceinline__ void headSlot(const float* ov, int* __restrict__ slot, int nb) {
+    const int t = threadIdx.x;
+    if (t < D / 4) {
+        const float y[4] = {ov[4 * t], ov[4 * t + 1], ov[4 * t + 2], ov[4 * t + 3]};
+        const Q8L o = quant8(y);
+        const int b = blockIdx.x * (D / 32) + (t >> 3), j = t & 7;
+        slot[b * 8 + j] = o.w;
+        if (j == 0) *reinterpret_cast<float2*>(slot + nb * 8 + 2 * b) = make_float2(o.d, (float)o.sum);
+    }
+}
+
 // out[i][h][:] of the chunk partials of (token i, head h) = blockIdx.x, in chunk order. The
 // partials of 16 chunks are loaded before they are merged (one memory round trip per 16 chunks).
 // slot (optional, one token): the head's D outputs also quantized per 32 into the per-32 slot of
@@ -1266,14 +1280,79 @@ __global__ __launch_bounds__(128) void flash_merge_kernel(const float* __restric
     }
     if (slot) {
         __syncthreads();
-        const int t = threadIdx.x;
-        if (t < D / 4) {  // eight lanes per block of 32, four values each
-            const float y[4] = {ov[4 * t], ov[4 * t + 1], ov[4 * t + 2], ov[4 * t + 3]};
-            const Q8L o = quant8(y);
-            const int b = blockIdx.x * (D / 32) + (t >> 3), j = t & 7;
-            slot[b * 8 + j] = o.w;
-            if (j == 0) *reinterpret_cast<float2*>(slot + nb * 8 + 2 * b) = make_float2(o.d, (float)o.sum);
+        headSlot<D>(ov, slot, nb);
+    }
+}
+
+// The same merge of more than 16 chunks, by 8 wavefronts: wavefront w merges chunks w, w + 8, .. (each lane D / 64 of
+// the outputs, 8 chunks' loads issued together) with a running maximum, and the 8 results are merged in LDS. A
+// chunk-order merge by one workgroup of 128 threads waits for a memory round trip per 16 chunks, one after the
+// other: at 128 chunks (a context of 8192, 32 heads of 128) it took 23.4 us, twice the attention itself; this takes
+// 3.9 us. Up to 16 chunks the kernel above waits once and is kept (its order of sums with it).
+constexpr int kMergeWaves = 8;
+template <int D>
+__global__ __launch_bounds__(64 * kMergeWaves) void flash_merge_wide_kernel(const float* __restrict__ part,
+                                                                            float* __restrict__ out, int nch,
+                                                                            int* __restrict__ slot, int nb) {
+    constexpr int E = D / 64, U = 8;
+    __shared__ float ov[kMergeWaves][D], ml[kMergeWaves][2];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const float* base = part + (size_t)blockIdx.x * nch * (D + 2);
+    float M = -INFINITY, L = 0.0f, O[E] = {};
+    for (int c0 = wave; c0 < nch; c0 += kMergeWaves * U) {
+        float mc[U], lc[U], oc[U][E];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {  // unconditional loads (chunks past nch reread the last)
+            const float* pc = base + (size_t)min(c0 + kMergeWaves * u, nch - 1) * (D + 2);
+            mc[u] = pc[D];
+            lc[u] = pc[D + 1];
+#pragma unroll
+            for (int e = 0; e < E; ++e) oc[u][e] = pc[lane + 64 * e];
         }
+        float m = M;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (c0 + kMergeWaves * u >= nch) mc[u] = -INFINITY;
+            m = fmaxf(m, mc[u]);
+        }
+        if (m == -INFINITY) continue;  // every position so far masked
+        const float f0 = exp2f((M - m) * kLog2e);
+        L *= f0;
+#pragma unroll
+        for (int e = 0; e < E; ++e) O[e] *= f0;
+        M = m;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const float f = exp2f((mc[u] - M) * kLog2e);
+            L += lc[u] * f;
+#pragma unroll
+            for (int e = 0; e < E; ++e) O[e] += oc[u][e] * f;
+        }
+    }
+#pragma unroll
+    for (int e = 0; e < E; ++e) ov[wave][lane + 64 * e] = O[e];
+    if (lane == 0) {
+        ml[wave][0] = M;
+        ml[wave][1] = L;
+    }
+    __syncthreads();
+    const int t = threadIdx.x;
+    if (t < D) {
+        float m = -INFINITY, l = 0.0f, o = 0.0f;
+#pragma unroll
+        for (int w = 0; w < kMergeWaves; ++w) m = fmaxf(m, ml[w][0]);
+#pragma unroll
+        for (int w = 0; w < kMergeWaves; ++w) {
+            const float f = ml[w][0] == -INFINITY ? 0.0f : exp2f((ml[w][0] - m) * kLog2e);
+            l += ml[w][1] * f;
+            o += ov[w][t] * f;
+        }
+        out[(size_t)blockIdx.x * D + t] = o / l;
+        ov[0][t] = o / l;  // (thread t alone reads and writes column t)
+    }
+    if (slot) {
+        __syncthreads();
+        headSlot<D>(ov[0], slot, nb);
     }
 }
 
@@ -1454,7 +1533,12 @@ int launchFlashDecode(const kcFlashDecodeArgs& a, hipStream_t s, int* slot, cons
     if (int e = fromHip(hipGetLastError(), "flash_decode_f16")) return e;
     if (slot && (d.N != 1 || (d.H * d.D) % 32)) return fromHip(hipErrorInvalidValue, "flash_decode_f16: slot of one token");
     const int nb = d.H * d.D / 32;
-    if (d.D == 128)
+    const dim3 wide(64 * kMergeWaves);
+    if (nch > 16 && d.D == 128)
+        hipLaunchKernelGGL(flash_merge_wide_kernel<128>, dim3(d.N * d.H), wide, 0, s, a.part, a.out, nch, slot, nb);
+    else if (nch > 16)
+        hipLaunchKernelGGL(flash_merge_wide_kernel<64>, dim3(d.N * d.H), wide, 0, s, a.part, a.out, nch, slot, nb);
+    else if (d.D == 128)
         hipLaunchKernelGGL(flash_merge_kernel<128>, dim3(d.N * d.H), dim3(128), 0, s, a.part, a.out, nch, slot, nb);
     else
         hipLaunchKernelGGL(flash_merge_kernel<64>, dim3(d.N * d.H), dim3(128), 0, s, a.part, a.out, nch, slot, nb);
