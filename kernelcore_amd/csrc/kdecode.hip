@@ -1284,75 +1284,72 @@ __global__ __launch_bounds__(128) void flash_merge_kernel(const float* __restric
     }
 }
 
-// The same merge of more than 16 chunks, by 8 wavefronts: wavefront w merges chunks w, w + 8, .. (each lane D / 64 of
-// the outputs, 8 chunks' loads issued together) with a running maximum, and the 8 results are merged in LDS. A
-// chunk-order merge by one workgroup of 128 threads waits for a memory round trip per 16 chunks, one after the
-// other: at 128 chunks (a context of 8192, 32 heads of 128) it took 23.4 us, twice the attention itself; this takes
-// 3.9 us. Up to 16 chunks the kernel above waits once and is kept (its order of sums with it).
-constexpr int kMergeWaves = 8;
+// The same merge of more than 16 chunks, the same bits: 8 wavefronts fetch 64 chunks' partials at a time into LDS (the
+// next 64's loads in flight meanwhile) with the running maximum's factors, and D threads run the chunk-order sums from
+// there: per chunk one product and one sum, the rescale a product with 1 where the maximum stays. The kernel above waits
+// for a memory round trip per 16 chunks, one after the other: at 128 chunks (a context of 8192, 32 heads of 128) 23.4
+// us, twice the attention itself; this takes 6.1.
+constexpr int kMergeChunks = 64, kMergeThreads = 512;
 template <int D>
-__global__ __launch_bounds__(64 * kMergeWaves) void flash_merge_wide_kernel(const float* __restrict__ part,
-                                                                            float* __restrict__ out, int nch,
-                                                                            int* __restrict__ slot, int nb) {
-    constexpr int E = D / 64, U = 8;
-    __shared__ float ov[kMergeWaves][D], ml[kMergeWaves][2];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+__global__ __launch_bounds__(kMergeThreads) void flash_merge_wide_kernel(const float* __restrict__ part,
+                                                                         float* __restrict__ out, int nch,
+                                                                         int* __restrict__ slot, int nb) {
+    constexpr int N = kMergeChunks * D / kMergeThreads;  // partial values a thread fetches per batch
+    __shared__ float po[kMergeChunks][D], fr[kMergeChunks], fc[kMergeChunks], lc[kMergeChunks], ov[D];
+    const int t = threadIdx.x, e = t % D, lane = t & 63;
     const float* base = part + (size_t)blockIdx.x * nch * (D + 2);
-    float M = -INFINITY, L = 0.0f, O[E] = {};
-    for (int c0 = wave; c0 < nch; c0 += kMergeWaves * U) {
-        float mc[U], lc[U], oc[U][E];
+    float o[N], m = 0.0f, l = 0.0f;
+    auto fetch = [&](int c0) {  // unconditional loads (chunks past nch reread the last)
 #pragma unroll
-        for (int u = 0; u < U; ++u) {  // unconditional loads (chunks past nch reread the last)
-            const float* pc = base + (size_t)min(c0 + kMergeWaves * u, nch - 1) * (D + 2);
-            mc[u] = pc[D];
-            lc[u] = pc[D + 1];
-#pragma unroll
-            for (int e = 0; e < E; ++e) oc[u][e] = pc[lane + 64 * e];
+        for (int u = 0; u < N; ++u) o[u] = base[(size_t)min(c0 + u * (kMergeThreads / D) + t / D, nch - 1) * (D + 2) + e];
+        if (t < 64) {
+            const float* pc = base + (size_t)min(c0 + lane, nch - 1) * (D + 2) + D;
+            m = pc[0];
+            l = pc[1];
         }
-        float m = M;
+    };
+    float M = -INFINITY, L = 0.0f, O = 0.0f;
+    fetch(0);
+    for (int c0 = 0; c0 < nch; c0 += kMergeChunks) {
+        if (c0) __syncthreads();  // the last batch has been summed
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            if (c0 + kMergeWaves * u >= nch) mc[u] = -INFINITY;
-            m = fmaxf(m, mc[u]);
+        for (int u = 0; u < N; ++u) po[u * (kMergeThreads / D) + t / D][e] = o[u];
+        if (t < 64) {
+            // lane = chunk: the running maximum before it and with it
+            const float own = c0 + lane < nch ? m : -INFINITY;
+            float run = own;
+#pragma unroll
+            for (int s = 1; s < 64; s <<= 1) {
+                const float v = __shfl_up(run, s);
+                if (lane >= s) run = fmaxf(run, v);
+            }
+            run = fmaxf(run, M);
+            float before = __shfl_up(run, 1);
+            if (lane == 0) before = M;
+            const bool live = own != -INFINITY;
+            fr[lane] = live && own > before ? exp2f((before - own) * kLog2e) : 1.0f;
+            fc[lane] = live ? exp2f((own - run) * kLog2e) : 0.0f;  // 0: every position of the chunk masked (its sums are 0)
+            lc[lane] = l;
+            M = __shfl(run, 63);
         }
-        if (m == -INFINITY) continue;  // every position so far masked
-        const float f0 = exp2f((M - m) * kLog2e);
-        L *= f0;
-#pragma unroll
-        for (int e = 0; e < E; ++e) O[e] *= f0;
-        M = m;
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const float f = exp2f((mc[u] - M) * kLog2e);
-            L += lc[u] * f;
-#pragma unroll
-            for (int e = 0; e < E; ++e) O[e] += oc[u][e] * f;
+        __syncthreads();
+        if (c0 + kMergeChunks < nch) fetch(c0 + kMergeChunks);
+        if (t < D) {
+#pragma unroll 8
+            for (int c = 0; c < kMergeChunks; ++c) {
+                const float r = fr[c], f = fc[c];
+                L = L * r + lc[c] * f;
+                O = O * r + po[c][t] * f;
+            }
         }
     }
-#pragma unroll
-    for (int e = 0; e < E; ++e) ov[wave][lane + 64 * e] = O[e];
-    if (lane == 0) {
-        ml[wave][0] = M;
-        ml[wave][1] = L;
-    }
-    __syncthreads();
-    const int t = threadIdx.x;
     if (t < D) {
-        float m = -INFINITY, l = 0.0f, o = 0.0f;
-#pragma unroll
-        for (int w = 0; w < kMergeWaves; ++w) m = fmaxf(m, ml[w][0]);
-#pragma unroll
-        for (int w = 0; w < kMergeWaves; ++w) {
-            const float f = ml[w][0] == -INFINITY ? 0.0f : exp2f((ml[w][0] - m) * kLog2e);
-            l += ml[w][1] * f;
-            o += ov[w][t] * f;
-        }
-        out[(size_t)blockIdx.x * D + t] = o / l;
-        ov[0][t] = o / l;  // (thread t alone reads and writes column t)
+        out[(size_t)blockIdx.x * D + t] = O / L;
+        ov[t] = O / L;
     }
     if (slot) {
         __syncthreads();
-        headSlot<D>(ov[0], slot, nb);
+        headSlot<D>(ov, slot, nb);
     }
 }
 
@@ -1533,7 +1530,7 @@ int launchFlashDecode(const kcFlashDecodeArgs& a, hipStream_t s, int* slot, cons
     if (int e = fromHip(hipGetLastError(), "flash_decode_f16")) return e;
     if (slot && (d.N != 1 || (d.H * d.D) % 32)) return fromHip(hipErrorInvalidValue, "flash_decode_f16: slot of one token");
     const int nb = d.H * d.D / 32;
-    const dim3 wide(64 * kMergeWaves);
+    const dim3 wide(kMergeThreads);
     if (nch > 16 && d.D == 128)
         hipLaunchKernelGGL(flash_merge_wide_kernel<128>, dim3(d.N * d.H), wide, 0, s, a.part, a.out, nch, slot, nb);
     else if (nch > 16)
