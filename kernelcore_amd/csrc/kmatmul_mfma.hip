@@ -1061,6 +1061,19 @@ bool wsRuns(bool q6) {
     return ws != 1 && !(ws == 3 && q6) && (path == 0 || path == 2);
 }
 
+// Whether Q6_K per-256 batches of nsb super-blocks run on the int8 kernel (from 16-byte aligned slots; options matmul_ws = 1,
+// 2, 3 keep the fp16 kernels).
+bool i8Runs(int nsb) {
+    const int path = option("matmul_path");
+    return (path == 0 || path == 2) && option("matmul_ws") == 0 && matmulI8Fits(nsb);
+}
+// ... and whether these parts over slots xq do (Q6_K alone).
+bool i8Group(const MmPart* parts, int nparts, const int* xq, int nsb) {
+    for (int i = 0; i < nparts; ++i)
+        if (!parts[i].q6) return false;
+    return xq && i8Runs(nsb) && (reinterpret_cast<uintptr_t>(xq) & 15) == 0;
+}
+
 int hWaves(long long wgs8) {
     const int o = option("matmul_waves");
     if (option("matmul_path") == 7 || o == 4) return 4;
@@ -1113,6 +1126,7 @@ int runMfmaH(const MmPart* parts, int nparts, const int* xq, int k, int ncols, i
     }
     g.nparts = nparts;
     g.ks = ks;
+    if (i8Group(parts, nparts, xq, nsb)) return launchMatmulI8(g, xq, nsb, ncols, s);
     // slots handed over (no quantizer-written fp16 operands) to Q4_K matrices: the producer
     // wavefronts convert them themselves, unless option matmul_ws = 2 (a conversion launch first,
     // as for the other kernels and for Q6_K)
@@ -1349,6 +1363,7 @@ bool matmulGroupSplitsQ6(const MmPart* parts, int nparts, int k, int ncols) {
     return mfmaWsFits(g, k / 256, ncols) && splitsQ6(g, nparts, k / 256);
 }
 
+bool matmulQ6ReadsSlots(int ncols, int k) { return ncols >= 64 && mfmaHUsable(ncols, k) && i8Runs(k / 256); }
 bool matmulGroupReadsActOnly(int ncols, int k) { return ncols >= 64 && mfmaHUsable(ncols, k); }
 
 int launchMatmulGroup(const MmPart* parts, int nparts, const int* xq, int k, int ncols, int ks, int* used_ks,
@@ -1359,6 +1374,10 @@ int launchMatmulGroup(const MmPart* parts, int nparts, const int* xq, int k, int
     if (nparts < 1 || nparts > 3 || ks < 1 || ks > 2 || k % 256 != 0) return fromHip(hipErrorInvalidValue, "matmul group");
     if (matmulGroupReadsActOnly(ncols, k)) {
         if (ks > k / 256) ks = 1;
+        if (i8Group(parts, nparts, xq, k / 256)) {  // (reads the slots alone, whether pre is given or not)
+            *used_ks = ks;
+            return runMfmaH(parts, nparts, xq, k, ncols, ks, nullptr, s);
+        }
         if (pre) {
             *used_ks = ks;
             return runMfmaH(parts, nparts, xq, k, ncols, ks, nullptr, s, pre, part_ks);

@@ -46,4 +46,10 @@ int launchMfmaWs(const MfmaGroup& g, int tiles, const void* act, const void* min
 bool mfmaWsSlotsFits(int nsb);
 int launchMfmaWsSlots(const MfmaGroup& g, int tiles, const int* xq, int nsb, int ncols, hipStream_t s);
 
+// The int8 kernel (kmatmul_i8.hip): Q6_K parts over the per-256 slots xq themselves (16-byte aligned), the group's split over
+// K. matmulI8Fits: slot rows of whole 16-byte pieces (k a multiple of 1024) and 32-bit offsets within a tile.
+bool matmulI8Fits(int nsb);
+int launchMatmulI8(MfmaGroup g, const int* xq, int nsb, int ncols, hipStream_t s);
+int cuCount();
+
 }  // namespace kcamd

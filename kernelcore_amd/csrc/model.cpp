@@ -417,7 +417,7 @@ int batchStep(kcModel_st* m, int n, hipStream_t s) {
                                             aE, yq));
         std::array<bool, 3> split{};  // (v may run in two K ranges: stored as v + v2)
         KI_TRY(batchProj(l, {KC_TENSOR_WQ, KC_TENSOR_WK, KC_TENSOR_WV}, {l.wq, l.wk, l.wv}, {m->q, m->k, m->v},
-                         {Q, KV, KV}, 3, m->slotEK, m->xn, E_, n, s, aE, {nullptr, nullptr, m->v2}, &split));
+                         {Q, KV, KV}, 3, sE, m->xn, E_, n, s, aE, {nullptr, nullptr, m->v2}, &split));
         // RoPE of q and k with the fp16 cache stores of k and v in one kernel, Qwen3's per-head q / k
         // norms in the same launch (option qk_fuse = 1: the norms as launches of their own)
         const bool fuse = c.qk_norm && kcamd::option("qk_fuse") != 1 && (c.head_dim == 64 || c.head_dim == 128);
@@ -440,7 +440,7 @@ int batchStep(kcModel_st* m, int n, hipStream_t s) {
         } else {
             KI_TRY(kcamd::launchQuantizeColsK(m->att, sQ, Q, n, s, aQ));
             const kcamd::MmPart op{l.wo, {m->o, m->o2}, E_, l.q6[KC_TENSOR_WO]};
-            KI_TRY(kcamd::launchMatmulGroup(&op, 1, m->slotQK, Q, n, kcamd::matmulKs(E_, Q, n, op.q6 != 0), &ks, s,
+            KI_TRY(kcamd::launchMatmulGroup(&op, 1, sQ, Q, n, kcamd::matmulKs(E_, Q, n, op.q6 != 0), &ks, s,
                                             aQ));
             o2 = ks == 2 ? m->o2 : nullptr;
         }
@@ -449,18 +449,22 @@ int batchStep(kcModel_st* m, int n, hipStream_t s) {
             KI_TRY(kcamd::launchAddNormQ8K(m->x, m->o, o2, m->x, l.ffn_norm, sE, E_, n, c.norm_eps, s, aE,
                                            f16_gu ? m->xn : nullptr));
             KI_TRY(batchProj(l, {KC_TENSOR_W_GATE, KC_TENSOR_W_UP, 0}, {l.wg, l.wu, nullptr},
-                             {m->gate, m->up, nullptr}, {c.n_ff, c.n_ff, 0}, 2, m->slotEK, m->xn, E_, n, s, aE));
+                             {m->gate, m->up, nullptr}, {c.n_ff, c.n_ff, 0}, 2, sE, m->xn, E_, n, s, aE));
             // SwiGLU straight into the quantized form (and into f32 when the down matrix is F16)
             const bool f16_d = l.f16[KC_TENSOR_W_DOWN];
-            kcSiluMulQ8FArgs sa{m->gate, m->up, f16_d ? m->sw : nullptr, sF, nullptr, c.n_ff, n};
-            KI_TRY(kcamd::launchSiluMulQ8KAct(sa, aF, s));
+            // (a Q6_K down matrix on the int8 kernel: the slots alone)
+            const bool slots = !f16_d && l.q6[KC_TENSOR_W_DOWN] && kcamd::matmulQ6ReadsSlots(n, c.n_ff);
+            int* qF = slots ? m->slotFK : sF;
+            const kcamd::ActF16* pF = slots ? nullptr : aF;
+            kcSiluMulQ8FArgs sa{m->gate, m->up, f16_d ? m->sw : nullptr, qF, nullptr, c.n_ff, n};
+            KI_TRY(kcamd::launchSiluMulQ8KAct(sa, pF, s));
             if (f16_d) {
                 KI_TRY(kcamd::launchMatmulF16(l.wd, m->sw, m->down, E_, c.n_ff, n, s));
                 down2 = nullptr;
             } else {
                 const kcamd::MmPart dp{l.wd, {m->down, m->down2}, E_, l.q6[KC_TENSOR_W_DOWN]};
-                KI_TRY(kcamd::launchMatmulGroup(&dp, 1, m->slotFK, c.n_ff, n, kcamd::matmulKs(E_, c.n_ff, n, dp.q6 != 0),
-                                                &ks, s, aF));
+                KI_TRY(kcamd::launchMatmulGroup(&dp, 1, qF, c.n_ff, n, kcamd::matmulKs(E_, c.n_ff, n, dp.q6 != 0), &ks, s,
+                                                pF));
                 down2 = ks == 2 ? m->down2 : nullptr;
             }
         } else {  // the last layer continues with the last token only
