@@ -310,7 +310,8 @@ __device__ __forceinline__ Q8L quant8(const float (&y)[4]) {
 // four passes of the workgroup): the per-32 sums of squares in element order as a chain through
 // the 8 lanes (each lane continues the running sum it receives from its left neighbour: the same
 // additions as one thread over 32 values), their total in block order, r, y = x * r * w and the
-// 8-lane quantization. The x / w words of every pass are loaded first (NormRegs8).
+// 8-lane quantization. The x / w words of every pass are loaded first (NormRegs8); mid() runs once
+// the sums of squares are in LDS (the matvec issues more of its weights there).
 typedef float f32x4v __attribute__((ext_vector_type(4)));
 template <int NP>
 struct NormRegs8 {
@@ -326,9 +327,9 @@ __device__ __forceinline__ void loadNorm8(NormRegs8<NP>& r, const float* x, cons
         r.w[p] = reinterpret_cast<const i32x4*>(w)[t];
     }
 }
-template <int NP>
+template <int NP, class F>
 __device__ __forceinline__ void stageNorm8(const Act& A, float* ss, const NormRegs8<NP>& st, int n, float eps,
-                                           int nsbp) {
+                                           int nsbp, F mid) {
     const int tid = threadIdx.x, nth = blockDim.x, nb = n / 32, nq = n / 4;
     const int j = tid & 7;
     const int np = (nq + nth - 1) / nth;  // passes (<= NP: the launchers check)
@@ -356,6 +357,7 @@ __device__ __forceinline__ void stageNorm8(const Act& A, float* ss, const NormRe
     }
     for (int b = nb + tid; b < nsbp * 8; b += nth) ss[b] = 0.0f;
     __syncthreads();
+    mid();
     // the total in block order; every 16-byte read issued before the adds (ss is zero past nb up
     // to a multiple of 32 inside nsbp * 8, and tot + 0 = tot)
     float tot = 0.0f;
@@ -445,6 +447,26 @@ __device__ __forceinline__ void dmvItems(const DmvArgs& a, int part, const Act& 
     const int kq = lane >> 4, r = lane & 15;
     const int ngroups = a.ngroups, ntmax = 2 * ngroups * kGroupSb;
     const int nitems = ns * ngroups;
+    auto item = [&](const Pieces<Q6, true>& w, int i) {
+        const int j = i % ns, g = i / ns;
+        const int s = g * kGroupSb + kq;
+        const uint32_t* c = reinterpret_cast<const uint32_t*>(w.c);
+        float* tt = terms + (j * 16 + r) * (ntmax + 4);  // one row's terms, contiguous
+        if (Q6) {
+            float t0, t1;
+            q6k_terms(c, w.dbits, A.xs + s * kXs, A.dx + 8 * s, A.isum + 8 * s, A.s16 + 8 * s, &t0, &t1);
+            tt[2 * s] = t0;
+            tt[2 * s + 1] = t1;
+        } else {
+            tt[s] = q4k_term(c, A.xs + s * kXs, A.dx + 8 * s, A.dsum + 8 * s);
+        }
+    };
+    // One item per wavefront, the usual plan: straight from the registers, so that each slab's products
+    // wait for that slab alone (through the loop's copies the first product waited for all of them).
+    if (wave + nw >= nitems) {
+        if (first_live) item(first, wave);
+        return;
+    }
     Pieces<Q6, true> cur = first;
     bool cur_live = first_live;
     for (int i = wave; i < nitems; i += nw) {
@@ -456,28 +478,20 @@ __device__ __forceinline__ void dmvItems(const DmvArgs& a, int part, const Act& 
             nxt_live = sn.live;
             if (nxt_live) nxt.load(sn.qw + ((size_t)sn.tile * ngroups + in / ns) * kSeg, lane);
         }
-        if (cur_live) {
-            const int j = i % ns, g = i / ns;
-            const int s = g * kGroupSb + kq;
-            const uint32_t* c = reinterpret_cast<const uint32_t*>(cur.c);
-            float* tt = terms + (j * 16 + r) * (ntmax + 4);  // one row's terms, contiguous
-            if (Q6) {
-                float t0, t1;
-                q6k_terms(c, cur.dbits, A.xs + s * kXs, A.dx + 8 * s, A.isum + 8 * s, A.s16 + 8 * s, &t0, &t1);
-                tt[2 * s] = t0;
-                tt[2 * s + 1] = t1;
-            } else {
-                tt[s] = q4k_term(c, A.xs + s * kXs, A.dx + 8 * s, A.dsum + 8 * s);
-            }
-        }
+        if (cur_live) item(cur, i);
         cur = nxt;
         cur_live = nxt_live;
     }
 }
 
+// The slabs of a wavefront's first item in the order they are issued, and computed, in: Q4_K as they lie,
+// Q6_K its first half's (the ql, qh and scales) first.
+constexpr int kFirst6[kQ6kSlabs] = {0, 1, 2, 3, 8, 9, 12, 4, 5, 6, 7, 10, 11};
+
 // N8: the norm prologue with 8 lanes per block of 32 (stageNorm8, at most two passes of the
-// workgroup), else one thread per block (stageNorm).
-template <int PRO, int EPI, bool N8, int PRE = 0>
+// workgroup), else one thread per block (stageNorm). PRE slabs of each wavefront's weights are issued
+// before the activations are staged, MID halfway through a stageNorm8, the others after it.
+template <int PRO, int EPI, bool N8, int PRE = kQ4kSlabs, int MID = 0>
 __global__ __launch_bounds__(EPI == kEpiSwiglu ? 768 : 512) void dmv_kernel(DmvArgs a) {
     extern __shared__ int4 lds4[];
     int* lds = reinterpret_cast<int*>(lds4);
@@ -515,41 +529,56 @@ __global__ __launch_bounds__(EPI == kEpiSwiglu ? 768 : 512) void dmv_kernel(DmvA
     if (PRO == kProNorm && N8) loadNorm8(nr8, a.x, a.nw, a.k);
     else if (PRO == kProNorm) loadNorm(nr, a.x, a.nw, a.k);
     else loadSlot(st, a.xq, a.xd, a.k / 256);
-    // The first item (wave < nw <= items always): 13 slabs and a Q6_K d read for either type
-    // with no branch (a Q4_K segment rereads its last slab, and its d address is slab 0). A dead
-    // tile reads tile 0. Issued before the staging, so that the item's weights stream in while
-    // the activations are staged (the staging waits for its own loads only) -- except in the
-    // SwiGLU workgroups, whose 28 MB of weights issued all at once queue the activations' small
-    // loads behind them: there the weights are issued once the activations are staged.
+    // The first item (wave < nw <= items always). Its first nine slabs are read for either type with
+    // no branch (a load under a branch gets a wait of its own), the others once the type's branch is
+    // taken; a dead tile reads tile 0.
+    // A CU holds about 40 KB of loads in flight: a wavefront that issues more waits at the issue, and
+    // the staging's barriers with it. The norm prologue's wavefronts (4-5 thousand cycles of staging) so
+    // issue a part before it, the next part halfway, the rest after; the barrier puts every wavefront's
+    // activation loads before any weights (they come back in order). Gate/up of 8192 x 2 rows, k 3072,
+    // 28 MB, 12 wavefronts per CU: 9.7 us with 9 slabs before (issue and staging 12300 cycles), 8.9 with 3,
+    // 8.2 with 3 and 3 halfway (7000, the weights 3400 later: the rate of HBM). The slot prologue is short:
+    // nine at once stay best there (down projection, 3072 x 8192: 7.4 us with 3 to 13).
     Pieces<true, true> f6;
     Pieces<false, true> f4;
-    bool first_live = false;
-    // slabs [LO, HI) of the first item (SwiGLU: PRE of them before the staging, the rest after)
     const Slot s0 = slotOf<EPI>(a, part, wave % ns);
-    const int seg = q6 ? kQ6kSeg : kQ4kSeg, nsl = q6 ? kQ6kSlabs : kQ4kSlabs;
+    const int seg = q6 ? kQ6kSeg : kQ4kSeg;
     const uint8_t* p0 = s0.qw + ((size_t)(s0.live ? s0.tile : 0) * a.ngroups + wave / ns) * seg;
-    first_live = s0.live;
     auto loadFirst = [&](auto lo, auto hi) {
 #pragma unroll
         for (int i = decltype(lo)::value; i < decltype(hi)::value; ++i)
-            f6.c[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p0 + min(i, nsl - 1) * 1024 + lane * 16));
-        if constexpr (decltype(hi)::value == kQ6kSlabs)
-            f6.dbits = *reinterpret_cast<const uint16_t*>(p0 + (q6 ? kQ6kSlabs * 1024 + lane * 2 : 0));
+            f4.c[i] = __builtin_nontemporal_load(
+                reinterpret_cast<const u32x4*>(p0 + (q6 ? kFirst6[i] : i) * 1024 + lane * 16));
     };
     using Lo = std::integral_constant<int, 0>;
-    using Pre = std::integral_constant<int, (EPI == kEpiSwiglu ? PRE : kQ6kSlabs)>;
-    using Hi = std::integral_constant<int, kQ6kSlabs>;
+    using Pre = std::integral_constant<int, PRE>;
+    using Mid = std::integral_constant<int, PRE + MID>;
+    using Hi = std::integral_constant<int, kQ4kSlabs>;
+    __builtin_amdgcn_sched_barrier(0);
+    if (PRO == kProNorm) __builtin_amdgcn_s_barrier();
     loadFirst(Lo{}, Pre{});
     __builtin_amdgcn_sched_barrier(0);
-    if (PRO == kProNorm && N8) stageNorm8(A, extra, nr8, a.k, a.eps, nsbp);
+    if (PRO == kProNorm && N8)
+        stageNorm8(A, extra, nr8, a.k, a.eps, nsbp, [&] {
+            __builtin_amdgcn_sched_barrier(0);
+            loadFirst(Pre{}, Mid{});
+            __builtin_amdgcn_sched_barrier(0);
+        });
     else if (PRO == kProNorm) stageNorm(A, extra, nr, a.k, a.eps, nsbp);
     else stageSlot(A, extra, st, a.k / 256, nsbp);
     __syncthreads();
-    if constexpr (EPI == kEpiSwiglu) loadFirst(Pre{}, Hi{});
+    loadFirst(Mid{}, Hi{});
+    if (q6) {
+        f6.dbits = *reinterpret_cast<const uint16_t*>(p0 + kQ6kSlabs * 1024 + lane * 2);
 #pragma unroll
-    for (int i = 0; i < kQ4kSlabs; ++i) f4.c[i] = f6.c[i];
-    if (q6) dmvItems<true, EPI>(a, part, A, terms, ns, f6, first_live);
-    else dmvItems<false, EPI>(a, part, A, terms, ns, f4, first_live);
+        for (int i = 0; i < kQ6kSlabs; ++i)
+            f6.c[kFirst6[i]] = i < kQ4kSlabs ? f4.c[i < kQ4kSlabs ? i : 0]
+                                             : __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(
+                                                   p0 + kFirst6[i] * 1024 + lane * 16));
+        dmvItems<true, EPI>(a, part, A, terms, ns, f6, s0.live);
+    } else {
+        dmvItems<false, EPI>(a, part, A, terms, ns, f4, s0.live);
+    }
     __syncthreads();
 
     const int nreal = q6 ? 2 * (a.k / 256) : a.k / 256;
@@ -565,10 +594,16 @@ __global__ __launch_bounds__(EPI == kEpiSwiglu ? 768 : 512) void dmv_kernel(DmvA
 #pragma unroll
             for (int k = 0; k < 8; ++k) {
                 const int u = u0 + 4 * k;
-                if (u < nreal) acc += q[k].x;
-                if (u + 1 < nreal) acc += q[k].y;
-                if (u + 2 < nreal) acc += q[k].z;
-                if (u + 3 < nreal) acc += q[k].w;
+                if (u + 4 <= nreal) {  // (a test per four terms: 64 terms 2570 -> 1600 cycles)
+                    acc += q[k].x;
+                    acc += q[k].y;
+                    acc += q[k].z;
+                    acc += q[k].w;
+                } else {
+                    if (u < nreal) acc += q[k].x;
+                    if (u + 1 < nreal) acc += q[k].y;
+                    if (u + 2 < nreal) acc += q[k].z;
+                }
             }
         }
         if (EPI == kEpiSwiglu) {
@@ -1433,30 +1468,29 @@ int launchDecodeMatvec(int pro, int epi, DmvArgs a, hipStream_t s) {
     const bool n8 = plan.n8;
     const size_t lds = plan.lds;
     const dim3 grid(wgs), block(64 * nw);
-#define KC_DMV(P, Q)                                                                                         \
-    if (pro == P && epi == Q && n8 == (P == kProNorm && Q == kEpiSwiglu))                                    \
-        hipLaunchKernelGGL((dmv_kernel<P, Q, P == kProNorm && Q == kEpiSwiglu>), grid, block, lds, s, a);     \
-    if (pro == P && epi == Q && n8 && P == kProNorm && Q != kEpiSwiglu)                                        \
-        hipLaunchKernelGGL((dmv_kernel<P, Q, true>), grid, block, lds, s, a);
-    // The SwiGLU workgroups issue 9 of the 13 slab loads of each wavefront's weights before the
-    // activations are staged and the rest after (config 4 decode, measured: 812 tok/s with all
-    // after, 819 with 3 or 6 before, 821 with 9, 803 with all 13: their 28 MB in flight then delay
-    // the activation loads). Option "swiglu_pre": 1-13 that many before, 14 none.
+#define KC_DMV(P, Q, N8) \
+    if (pro == P && epi == Q && n8 == N8) hipLaunchKernelGGL((dmv_kernel<P, Q, N8>), grid, block, lds, s, a);
+    // The slabs issued before and during the norm prologue (8 lanes per block): see the kernel. Option
+    // "swiglu_pre": 1-13 that many before in the SwiGLU workgroups (in steps of three), 14 none.
     const int po = option("swiglu_pre");
-    const int pre = epi != kEpiSwiglu ? 0 : (po == 0 ? 9 : (po >= 14 ? 0 : po));
-    if (pre > 0 && pro == kProNorm && epi == kEpiSwiglu && n8) {
-        if (pre <= 3) hipLaunchKernelGGL((dmv_kernel<kProNorm, kEpiSwiglu, true, 3>), grid, block, lds, s, a);
-        else if (pre <= 6) hipLaunchKernelGGL((dmv_kernel<kProNorm, kEpiSwiglu, true, 6>), grid, block, lds, s, a);
-        else if (pre <= 9) hipLaunchKernelGGL((dmv_kernel<kProNorm, kEpiSwiglu, true, 9>), grid, block, lds, s, a);
-        else hipLaunchKernelGGL((dmv_kernel<kProNorm, kEpiSwiglu, true, 13>), grid, block, lds, s, a);
+    if (pro == kProNorm && epi == kEpiSwiglu && n8) {
+        if (po == 0) hipLaunchKernelGGL((dmv_kernel<kProNorm, kEpiSwiglu, true, 3, 3>), grid, block, lds, s, a);
+        else if (po >= 14) hipLaunchKernelGGL((dmv_kernel<kProNorm, kEpiSwiglu, true, 0>), grid, block, lds, s, a);
+        else if (po <= 3) hipLaunchKernelGGL((dmv_kernel<kProNorm, kEpiSwiglu, true, 3>), grid, block, lds, s, a);
+        else if (po <= 6) hipLaunchKernelGGL((dmv_kernel<kProNorm, kEpiSwiglu, true, 6>), grid, block, lds, s, a);
+        else hipLaunchKernelGGL((dmv_kernel<kProNorm, kEpiSwiglu, true, 9>), grid, block, lds, s, a);
         return fromHip(hipGetLastError(), "decode matvec");
     }
-    KC_DMV(kProSlot, kEpiStore)
-    KC_DMV(kProSlot, kEpiResid)
-    KC_DMV(kProNorm, kEpiStore)
-    KC_DMV(kProNorm, kEpiResid)
-    KC_DMV(kProNorm, kEpiSwiglu)
-    KC_DMV(kProSlot, kEpiSwiglu)
+    if (pro == kProNorm && epi == kEpiStore && n8) {  // (q / k / v, 5120 x 3072: 6.7 us with 9 before, 6.4 with 5 and 4)
+        hipLaunchKernelGGL((dmv_kernel<kProNorm, kEpiStore, true, 5, 4>), grid, block, lds, s, a);
+        return fromHip(hipGetLastError(), "decode matvec");
+    }
+    KC_DMV(kProSlot, kEpiStore, false)
+    KC_DMV(kProSlot, kEpiResid, false)
+    KC_DMV(kProSlot, kEpiSwiglu, false)
+    KC_DMV(kProNorm, kEpiStore, false)
+    KC_DMV(kProNorm, kEpiResid, false)
+    KC_DMV(kProNorm, kEpiResid, true)
 #undef KC_DMV
     return fromHip(hipGetLastError(), "decode matvec");
 }
