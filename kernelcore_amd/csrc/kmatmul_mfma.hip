@@ -1376,7 +1376,7 @@ int launchMatmulGroup(const MmPart* parts, int nparts, const int* xq, int k, int
         if (ks > k / 256) ks = 1;
         if (i8Group(parts, nparts, xq, k / 256)) {  // (reads the slots alone, whether pre is given or not)
             *used_ks = ks;
-            return runMfmaH(parts, nparts, xq, k, ncols, ks, nullptr, s);
+            return runMfmaH(parts, nparts, xq, k, ncols, ks, nullptr, s, nullptr, part_ks);
         }
         if (pre) {
             *used_ks = ks;
