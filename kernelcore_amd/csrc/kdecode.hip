@@ -1319,18 +1319,20 @@ __global__ __launch_bounds__(128) void flash_merge_kernel(const float* __restric
     }
 }
 
-// The same merge of more than 16 chunks, the same bits: 8 wavefronts fetch 64 chunks' partials at a time into LDS (the
-// next 64's loads in flight meanwhile) with the running maximum's factors, and D threads run the chunk-order sums from
-// there: per chunk one product and one sum, the rescale a product with 1 where the maximum stays. The kernel above waits
-// for a memory round trip per 16 chunks, one after the other: at 128 chunks (a context of 8192, 32 heads of 128) 23.4
-// us, twice the attention itself; this takes 6.1.
+// The same merge of more than 16 chunks, the same bits: 8 wavefronts fetch 64 chunks' partials at a time (the next 64's
+// loads in flight meanwhile), one forms the running maximum's factors, all multiply the partials by them into LDS, and D
+// threads run the chunk-order sums from there: the rescale (a product with 1 where the maximum stays) and one sum per chunk.
+// The kernel above waits for a memory round trip per 16 chunks, one after the other: at 128 chunks (a context of 8192, 32
+// heads of 128) 23.4 us, twice the attention itself; this takes 6.1.
+// A dead chunk (every position masked, or past nch) adds -0, which changes no sum, whatever its partials hold: the sum of
+// 0 * v over masked positions is NaN where v is infinite or NaN, so a factor of 0 would not keep it out.
 constexpr int kMergeChunks = 64, kMergeThreads = 512;
 template <int D>
 __global__ __launch_bounds__(kMergeThreads) void flash_merge_wide_kernel(const float* __restrict__ part,
                                                                          float* __restrict__ out, int nch,
                                                                          int* __restrict__ slot, int nb) {
     constexpr int N = kMergeChunks * D / kMergeThreads;  // partial values a thread fetches per batch
-    __shared__ float po[kMergeChunks][D], fr[kMergeChunks], fc[kMergeChunks], lc[kMergeChunks], ov[D];
+    __shared__ float po[kMergeChunks][D], fr[kMergeChunks], fc[kMergeChunks], lf[kMergeChunks], ov[D];
     const int t = threadIdx.x, e = t % D, lane = t & 63;
     const float* base = part + (size_t)blockIdx.x * nch * (D + 2);
     float o[N], m = 0.0f, l = 0.0f;
@@ -1347,8 +1349,6 @@ __global__ __launch_bounds__(kMergeThreads) void flash_merge_wide_kernel(const f
     fetch(0);
     for (int c0 = 0; c0 < nch; c0 += kMergeChunks) {
         if (c0) __syncthreads();  // the last batch has been summed
-#pragma unroll
-        for (int u = 0; u < N; ++u) po[u * (kMergeThreads / D) + t / D][e] = o[u];
         if (t < 64) {
             // lane = chunk: the running maximum before it and with it
             const float own = c0 + lane < nch ? m : -INFINITY;
@@ -1363,18 +1363,26 @@ __global__ __launch_bounds__(kMergeThreads) void flash_merge_wide_kernel(const f
             if (lane == 0) before = M;
             const bool live = own != -INFINITY;
             fr[lane] = live && own > before ? exp2f((before - own) * kLog2e) : 1.0f;
-            fc[lane] = live ? exp2f((own - run) * kLog2e) : 0.0f;  // 0: every position of the chunk masked (its sums are 0)
-            lc[lane] = l;
+            const float f = live ? exp2f((own - run) * kLog2e) : -1.0f;  // -1: a dead chunk
+            fc[lane] = f;
+            lf[lane] = live ? l * f : -0.0f;
             M = __shfl(run, 63);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < N; ++u) {
+            const int c = u * (kMergeThreads / D) + t / D;
+            const float f = fc[c];
+            po[c][e] = f < 0.0f ? -0.0f : o[u] * f;
         }
         __syncthreads();
         if (c0 + kMergeChunks < nch) fetch(c0 + kMergeChunks);
         if (t < D) {
 #pragma unroll 8
             for (int c = 0; c < kMergeChunks; ++c) {
-                const float r = fr[c], f = fc[c];
-                L = L * r + lc[c] * f;
-                O = O * r + po[c][t] * f;
+                const float r = fr[c];
+                L = L * r + lf[c];
+                O = O * r + po[c][t];
             }
         }
     }
