@@ -37,14 +37,16 @@ typedef __amdgpu_buffer_rsrc_t Rsrc;
 constexpr int kWaves = 4;  // wavefronts per workgroup, 32 weight rows each
 constexpr int kRows = 32 * kWaves;
 // LDS: two stages of a super-block's int8 activations [column][16 chunks of 16 B]; two groups of four super-blocks'
-// column scales [column][4] (fetched per super-block they touched a cache line per column each time).
+// column scales [column][4] (fetched per super-block they touched a cache line per column each time); zeros as the scales of
+// the combine ahead of a range's first super-block (which adds 0: times a column's own scale that is NaN if it is infinite).
 template <int NB>
 struct Stage {
     static constexpr int kCols = 32 * NB;
     static constexpr int kBytes = kCols * 256;
     static constexpr int kXd = 2 * kBytes;
     static constexpr int kXdGroup = kCols * 16;
-    static constexpr int kLds = kXd + 2 * kXdGroup;
+    static constexpr int kZero = kXd + 2 * kXdGroup;
+    static constexpr int kLds = kZero + 32 * 16;
 };
 
 __device__ __forceinline__ Rsrc bufRes(const void* p, uint32_t bytes) {
@@ -185,6 +187,7 @@ __device__ __forceinline__ void i8Tile(char* lds, const uint8_t* __restrict__ qw
     const i32x16 zero = {};
     stage(0, sb0);
     scaleGroup(sb0 >> 2);
+    if (tid < 128) reinterpret_cast<float*>(lds + G::kZero)[tid] = 0.0f;
     raw.load(rw, sb0, lane, tileB);
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
@@ -195,10 +198,11 @@ __device__ __forceinline__ void i8Tile(char* lds, const uint8_t* __restrict__ qw
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
     __syncthreads();
     const int nt = sb1 - sb0;
+    const float* xdp = reinterpret_cast<const float*>(lds + G::kZero) + 16 * h - (NB - 1) * 128;  // the previous super-block's
     for (int t = 0; t < nt; ++t) {
         const int s = sb0 + t, sn = t + 1 < nt ? s + 1 : s;  // (past the range: the last one again, unused)
         const char* buf = lds + (t & 1) * G::kBytes;
-        const float *xd = xdOf(s), *xdp = xdOf(t ? s - 1 : s);
+        const float* xd = xdOf(s);
         stage(t + 1, sn);
         if ((s & 3) == 3) scaleGroup((s >> 2) + 1);
         raw.load(rw, sn, again(tid) & 63, tileB);
@@ -238,6 +242,7 @@ __device__ __forceinline__ void i8Tile(char* lds, const uint8_t* __restrict__ qw
         unpackHalf(raw, h, 7, 0, op);
         unpackHalf(raw, h, 7, 1, op);
         dp = d;
+        xdp = xd;
         d = f16(raw.d);
         asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
         __syncthreads();  // this stage read, the next one loaded

@@ -46,6 +46,28 @@ def test_int8_prefill_sums_past_24_bits():
     check(w, x, y, rows, k, ncols)
 
 
+@pytest.mark.parametrize("rows,ncols", [(48, 64), (16400, 200)])
+def test_int8_prefill_infinite_column_scale(rows, ncols):
+    """A column whose slot carries an infinite scale gives the oracle's infinities (64 and 128 columns per workgroup, the
+    first super-block of each K range; columns of every block of 32), and leaves the others alone."""
+    k = 1024
+    w, x = kq.random_blocks("q6k", rows, k, seed=9), kq.randn(k * ncols, 4, 1.5)
+    q = oracle_slots(x, k, ncols, True)
+    at = {5: 0, 40: 0, 41: 2, 63: 1} | ({100: 0, 127: 2, 130: 0, 199: 0} if ncols == 200 else {})
+    for c, s in at.items():
+        q.reshape(ncols, -1)[c, k // 4 + s] = np.float32(np.inf).view(np.int32)
+    stream, slots, y = kc.upload_weights("q6k", w, rows, k), kc.Buffer.of(q), kc.Buffer(4 * rows * ncols)
+    kc.launch("matmul_q6k_q8kx8", kc.MatmulKQ8Args(stream.ptr, slots.ptr, y.ptr, None, rows, k, ncols, 8))
+    got, want = y.download(np.float32).reshape(ncols, rows), np.zeros(rows * ncols, np.float32)
+    O.kco_matmul_q6k_q8k(w, q, want, rows, k, ncols)
+    want = want.reshape(ncols, rows)
+    assert np.isinf(want[list(at)]).mean() > 0.9
+    assert np.array_equal(got[list(at)], want[list(at)], equal_nan=True)
+    assert np.isfinite(np.delete(got, list(at), 0)).all()
+    for b in (stream, slots, y):
+        b.free()
+
+
 def check(w, x, y, rows, k, ncols):
     cols = np.unique(np.r_[0, ncols // 2, ncols - 1, np.arange(0, ncols, 67)])
     xs = np.ascontiguousarray(x.reshape(ncols, k)[cols]).reshape(-1)
