@@ -301,9 +301,10 @@ int launchMatmulI8(MfmaGroup g, const int* xq, int nsb, int ncols, hipStream_t s
         tiles += (g.p[i].rows + kRows - 1) / kRows;
     }
     // 128 columns per workgroup unpack each weight half as often, but pay only where two such workgroups per CU
-    // have work (k 3072, 512 columns: 16384 rows 58.4 us against 79 with 64; 8192 rows 45 against 39)
+    // have work (k 3072, 512 columns: 16384 rows 58.4 us against 79 with 64; 8192 rows 45 against 39) and more than 64
+    // columns (64 columns, half a tile of padding: 128256 x 3072 134 us against 111)
     const long long wgs = (long long)tiles * ((ncols + 127) / 128) * g.ks;
-    return wgs >= 2LL * cuCount() ? launch<4>(g, tiles, xq, nsb, ncols, s) : launch<2>(g, tiles, xq, nsb, ncols, s);
+    return ncols > 64 && wgs >= 2LL * cuCount() ? launch<4>(g, tiles, xq, nsb, ncols, s) : launch<2>(g, tiles, xq, nsb, ncols, s);
 }
 
 }  // namespace kcamd
