@@ -9,13 +9,14 @@
 // computing NC columns from one load of its weights, and the per-row sum of super-block terms
 // done in registers in super-block order (the four lanes of a row pass their terms with
 // cross-lane reads, in order), which keeps every column bit-identical to the reference. It serves
-// the per-32 names and single columns; per-256 batches go to the MFMA kernels (kmatmul_short.hip, and
-// from 64 columns the prefill kernels).
+// the per-32 names, single columns and two (at times three) columns of a tall matrix; per-256 batches go to the
+// MFMA kernels (kmatmul_short.hip, and from 64 columns the prefill kernels).
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
 
 #include "internal.hpp"
+#include "kmatmul_mfma.hpp"
 #include "kmatmul_short.hpp"
 #include "kquant.hpp"
 #include "kquant_device.hpp"
@@ -161,8 +162,24 @@ int launchMatmulCols(bool q6k, bool per256, const kcMatmulKQ8Args& a, hipStream_
     return per256 ? pickCols<false, true>(a, s) : pickCols<false, false>(a, s);
 }
 
+// Two columns leave 14 of the short-batch kernel's 16 empty, and where a tall matrix fills the GPU whatever the kernel, the
+// column tiles' wavefront per 16 rows does less per weight: a workgroup of 64 rows, so they are at their best with nearly whole
+// numbers of workgroups per CU. us, column tiles / short batch: Q6_K 128256 x 1024 34 / 44, x 4096 96 / 116, 16384 x 4096
+// 23.6 / 25.5 (but 20480 x 4096, 1.25 workgroups per CU, 31.6 / 28.6); Q4_K 49152 x 4096 38 / 43, 16384 x 1024 14.8 / 15.8 (but
+// 65536 x 4096 56 / 53). Up to 512 values a wavefront has too little to do, and the short-batch kernel stays faster. Three
+// columns: Q6_K 128256 x 1024 38.5 / 44.3, x 2048 64 / 65; Q4_K 49152 x 1024 20.5 / 21.7, 65536 x 1024 25.0 / 24.0.
+static bool colsRuns(bool q6k, int rows, int k, int ncols) {
+    if (k <= 512 || ncols > 3) return false;
+    const double perCu = tilesOf(rows) / 4.0 / cuCount();
+    const bool whole = perCu > 1.7 && perCu <= 3 && perCu / __builtin_ceil(perCu) > 0.83;  // nearly two or three
+    if (ncols == 3) return k <= 1024 && (whole || (q6k && perCu > 3.5));
+    if (k <= 1024) return perCu > 0.55;
+    if (q6k) return perCu > 1.6 || (perCu <= 1 && perCu > (k <= 2048 ? 0.55 : 0.8));
+    return whole || perCu >= 5;
+}
+
 int launchMatmulFew(bool q6k, bool per256, const kcMatmulKQ8Args& a, hipStream_t s) {
-    if (per256 && matmulShortRuns(a.k, a.ncols))
+    if (per256 && matmulShortRuns(a.k, a.ncols) && !colsRuns(q6k, a.rows, a.k, a.ncols))
         return launchMatmulShort(ShortGroup{{{reinterpret_cast<const uint8_t*>(a.qw), a.y, a.rows, q6k, 0}}, 1}, a.xq, a.k,
                                  a.ncols, s);
     return launchMatmulCols(q6k, per256, a, s);

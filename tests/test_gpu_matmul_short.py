@@ -25,6 +25,7 @@ def runtime():
 @pytest.mark.parametrize("rows,k,ncols,shift", [
     (8, 256, 2, 0), (24, 1024, 16, 0), (40, 1024, 17, 0), (200, 1280, 33, 0), (1000, 2048, 63, 0), (16, 4096, 15, 0),
     (136, 12288, 40, 0), (24, 16384, 50, 0), (72, 8192, 62, 0), (48, 1024, 31, 1),
+    (9224, 1024, 2, 0), (13320, 2304, 2, 1),  # column tiles
 ])
 def test_short_batch_is_bit_exact(qtype, rows, k, ncols, shift):
     print(f"short batch {qtype} {rows}x{k} ncols={ncols} shift={shift}", flush=True)

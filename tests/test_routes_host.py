@@ -71,3 +71,16 @@ def test_q6k_prefill_column_tile(routes):
     got = routes([("matmul", ("q6k", rows, 3072, n)) for rows, n in ((128256, 64), (65536, 64), (128256, 65), (16384, 512), (512, 65))])
     assert [g[0][0] for g in got] == ["matmul_i8_kernel,2", "matmul_i8_kernel,2", "matmul_i8_kernel,4", "matmul_i8_kernel,4",
                                       "matmul_i8_kernel,2"]
+
+
+def test_two_columns_of_a_tall_matrix(routes):
+    """The column tiles where they were measured faster (one line of sizes on either side), the short-batch kernel else."""
+    cols = [("q6k", 128256, 1024, 2), ("q6k", 128256, 4096, 2), ("q6k", 16384, 4096, 2), ("q6k", 10240, 2048, 2),
+            ("q6k", 65536, 1024, 3), ("q4k", 16384, 1024, 2), ("q4k", 49152, 4096, 2), ("q4k", 128256, 2048, 2),
+            ("q4k", 32768, 1024, 3)]
+    short = [("q6k", 128256, 512, 2), ("q6k", 20480, 4096, 2), ("q6k", 8192, 1024, 2), ("q6k", 10240, 4096, 2),
+             ("q6k", 128256, 2048, 3), ("q6k", 128256, 1024, 4), ("q4k", 65536, 4096, 2), ("q4k", 8192, 3072, 2),
+             ("q4k", 65536, 1024, 3), ("q4k", 16384, 4096, 2)]
+    got = routes([("matmul", c) for c in cols + short])
+    names = [g[0][0].split(",")[0] for g in got]
+    assert names == ["matmul_cols_kernel"] * len(cols) + ["matmul_short_kernel"] * len(short)
