@@ -1387,7 +1387,7 @@ int launchMatmulGroup(const MmPart* parts, int nparts, const int* xq, int k, int
             return runMfmaH(parts, nparts, xq, k, ncols, ks, act, s, nullptr, part_ks);
         }
     }
-    if (nparts > 1 && option("matmul_path") == 0 && matmulShortRuns(k, ncols)) {  // one launch for the group
+    if (nparts > 1 && ncols < 64 && option("matmul_path") == 0 && matmulShortRuns(k, ncols)) {  // one launch for the group
         ShortGroup g{};
         g.nparts = nparts;
         for (int i = 0; i < nparts; ++i)

@@ -11,6 +11,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 
 CHILD = r"""
 import ctypes as C, json, re, sys
+import numpy as np
 stub = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
 stub.stub_record.restype = C.c_char_p
 import kernelcore_amd as kc
@@ -44,13 +45,39 @@ def f16(rows, k, ncols):
     return r
 
 
-print(json.dumps([globals()[name](*args) for name, args in json.loads(sys.argv[2])]))
+def model(n, types={}, options={}, no_scratch=0, **cfg):
+    # a prompt of n tokens on a two-layer driver (the last layer's FFN runs on one token); no_scratch: streams' staging
+    # buffers cannot grow (as while a stream captures)
+    cfg = dict(dict(n_layer=2, n_embd=1024, n_head=8, n_head_kv=2, head_dim=128, n_ff=2048, n_vocab=512, max_ctx=n,
+                    max_batch=n, norm_eps=1e-5, rope_theta=1e4), **cfg)
+    m = kc.Model(**cfg)
+    for name, t in kc.TENSORS.items():
+        if name in ("q_norm", "k_norm", "rope_freqs"):
+            continue
+        for layer in (-1,) if name in ("token_embd", "output_norm", "output") else (0, 1):
+            _, rows, k, nbytes = m.tensor_info(name, layer)
+            if name in types:
+                m.set_tensor(name, layer, np.zeros(rows * (k // 256) * {"q4k": 144, "q6k": 210}[types[name]], np.uint8), types[name])
+            else:
+                m.set_tensor(name, layer, np.zeros(nbytes, np.uint8))
+    for o, v in options.items():
+        kc.set_option(o, v)
+    stub.stub_capturing(no_scratch)
+    r = launched(lambda: m.forward(np.zeros(n, np.int32)))
+    stub.stub_capturing(0)
+    for o in options:
+        kc.set_option(o, 0)
+    m.close()
+    return r
+
+
+print(json.dumps([globals()[name](*args, **kw) for name, args, kw in json.loads(sys.argv[2])]))
 """
 
 
 @pytest.fixture(scope="module")
 def routes(tmp_path_factory):
-    """routes([(function, arguments)]): for each call its launches, [kernel, gridx, gridy, gridz, blockx]."""
+    """routes([(function, arguments[, keywords])]): for each call its launches, [kernel, gridx, gridy, gridz, blockx]."""
     import json
 
     lib = str(tmp_path_factory.mktemp("stub") / "libhipstub.so")
@@ -58,7 +85,7 @@ def routes(tmp_path_factory):
                     os.path.join(HERE, "hip_stub", "hip_stub.cpp"), "-o", lib], check=True)
 
     def run(calls):
-        r = subprocess.run([sys.executable, "-c", CHILD, lib, json.dumps(calls)], cwd=os.path.dirname(HERE), text=True,
+        r = subprocess.run([sys.executable, "-c", CHILD, lib, json.dumps([(*c, {})[:3] for c in calls])], cwd=os.path.dirname(HERE), text=True,
                            capture_output=True)
         assert r.returncode == 0, r.stderr[-2000:]
         return json.loads(r.stdout.splitlines()[-1])
@@ -84,3 +111,13 @@ def test_two_columns_of_a_tall_matrix(routes):
     got = routes([("matmul", c) for c in cols + short])
     names = [g[0][0].split(",")[0] for g in got]
     assert names == ["matmul_cols_kernel"] * len(cols) + ["matmul_short_kernel"] * len(short)
+
+
+def test_unstaged_batches_keep_the_prefill_kernel(routes):
+    """64 columns and more that cannot be staged run on the prefill kernel that stages nothing, not on the short-batch one:
+    past the fp16 layout's 32-bit offsets (a down projection of 16384 columns of 131072 values), and with no staging buffer."""
+    down, groups = routes([("model", [16384], dict(types={"w_down": "q4k"}, n_embd=256, n_head=2, n_head_kv=2, n_ff=131072)),
+                           ("model", [80], dict(types={"w_down": "q4k"}, options={"prefill_act": 1}, no_scratch=1))])
+    for got, count in ((down, 1), (groups, 2 * 4 + 2 + 1)):  # (q / k / v and o of two layers, gate / up and down of one)
+        names = [g[0].split(",")[0] for g in got if g[0].startswith("matmul_")]
+        assert "matmul_short_kernel" not in names and names.count("matmul_kq_mfma8_kernel") == count, names
