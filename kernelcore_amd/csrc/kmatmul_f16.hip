@@ -20,6 +20,7 @@
 // MFMA's accumulation): within the 1e-3 relative bar, not bit-identical.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 
 #include "internal.hpp"
@@ -257,14 +258,19 @@ __global__ __launch_bounds__(256) void mmf16_simple_kernel(const uint32_t* __res
 
 }  // namespace
 
+// Columns of one launch (the grid's second dimension).
+constexpr int kMaxCols = 1 << 20;
+
 int launchMatmulF16(const void* w, const float* x, float* y, int rows, int k, int ncols, hipStream_t s) {
     if (rows <= 0 || rows % 8 || k <= 0 || k % 2 || ncols <= 0)
         return fromHip(hipErrorInvalidValue, "matmul_f16: shape");
     const uint16_t* wh = static_cast<const uint16_t*>(w);
     // the vector kernels read 16 bytes at a time: w and x 16-byte aligned (hipMalloc gives 256)
     const bool a16 = ((reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(x)) & 15) == 0;
-    if (a16 && k % 8 == 0 && (ncols <= 8 || k % 16)) {
-        // columns in launches of at most 8 (only when k % 16 != 0 rules out the MFMA kernel)
+    // a tile's 32-bit byte offsets (past them at most 63 rows and columns)
+    const bool wide = (unsigned long long)k * 128 >= (1ull << 32);
+    if (a16 && k % 8 == 0 && (ncols <= 8 || k % 16 || wide)) {
+        // columns in launches of at most 8
         for (int c0 = 0; c0 < ncols; c0 += 8) {
             const int nc = ncols - c0 < 8 ? ncols - c0 : 8;
             const dim3 grid((rows / 2 + 3) / 4), block(256);
@@ -275,8 +281,11 @@ int launchMatmulF16(const void* w, const float* x, float* y, int rows, int k, in
             else if (nc <= 4) hipLaunchKernelGGL(mmf16_vec_kernel<4>, grid, block, 0, s, wh, xc, yc, rows, k, nc);
             else hipLaunchKernelGGL(mmf16_vec_kernel<8>, grid, block, 0, s, wh, xc, yc, rows, k, nc);
         }
-    } else if (a16 && k % 16 == 0 && (unsigned long long)k * 128 < (1ull << 32) && ncols <= 1 << 20) {
-        // (a tile's 32-bit byte offsets, the grid's second dimension)
+    } else if (a16 && k % 16 == 0 && ncols > kMaxCols) {
+        for (int c0 = 0; c0 < ncols; c0 += kMaxCols)
+            if (int e = launchMatmulF16(w, x + (size_t)c0 * k, y + (size_t)c0 * rows, rows, k, std::min(kMaxCols, ncols - c0), s))
+                return e;
+    } else if (a16 && k % 16 == 0) {
         // the smallest tile whose workgroups run at once on the 256 CUs (a second round costs more than a larger
         // tile: 1024 x 4096, 77 columns 12.4 us on 16 x 16 (320 workgroups), 9.9 us on 32 x 16 (160), 11.3 us on
         // 64 x 16 (80)), else the largest (512 columns: 18.7 us on 64 x 32, 22.5 us on 64 x 16); three stages where they

@@ -121,3 +121,13 @@ def test_unstaged_batches_keep_the_prefill_kernel(routes):
     for got, count in ((down, 1), (groups, 2 * 4 + 2 + 1)):  # (q / k / v and o of two layers, gate / up and down of one)
         names = [g[0].split(",")[0] for g in got if g[0].startswith("matmul_")]
         assert "matmul_short_kernel" not in names and names.count("matmul_kq_mfma8_kernel") == count, names
+
+
+def test_f16_limits(routes):
+    """Past a launch's columns and a tile's offsets matmul_f16 keeps kernels of whole wavefronts, not the one thread per
+    output of unaligned rows."""
+    got = routes([("f16", (8, 512, n)) for n in (1 << 20, (1 << 20) + 1, (2 << 20) + 70)]
+                 + [("f16", (8, k, 9)) for k in ((1 << 25) - 16, 1 << 25)])
+    names = [[g[0].split(",")[0] for g in c] for c in got]
+    assert names == [["mmf16_mfma_kernel"], ["mmf16_mfma_kernel", "mmf16_vec_kernel"], ["mmf16_mfma_kernel"] * 3,
+                     ["mmf16_mfma_kernel"], ["mmf16_vec_kernel"] * 2]
