@@ -10,7 +10,8 @@
 //   * ncols <= 8 (decode): one wavefront per 2 rows; each lane multiplies 8 consecutive values of
 //     a row with the same 8 values of every column, the partial sums are reduced across the 64
 //     lanes. HBM-bound (2 bytes per weight).
-//   * ncols > 8: v_mfma_f32_16x16x32_f16, K split over the wavefronts of a workgroup. The weights
+//   * ncols > 8: v_mfma_f32_16x16x32_f16, K split over the wavefronts of a workgroup (a tile
+//     per wavefront where the rows are too short for that). The weights
 //     are exact fp16 operands; each activation is split into hi = fp16(x) and lo = fp16(x - hi)
 //     and every product runs as two MFMAs (f32 accumulation), within about 2^-22 of the fp32
 //     product (a single fp16 rounding of x would be 2^-11).
@@ -24,6 +25,7 @@
 #include <cstdint>
 
 #include "internal.hpp"
+#include "kmatmul_mfma.hpp"
 #include "launch.hpp"
 
 namespace kcamd {
@@ -240,6 +242,82 @@ __global__ __launch_bounds__(64 * kF16Waves) void mmf16_mfma_kernel(const uint16
     f16Tile<T, C, S>(lds4, w, x, y, rows, k, ncols);
 }
 
+// ---- ncols > 8, k % 16 == 0, short rows: a workgroup of 4 wavefronts covers 64 rows x 64 columns, each wavefront 32 x 32 of
+// them (2 x 2 blocks, the operands and results laid out as above, straight from memory) over the whole row, 32 values at a
+// time from zero and added in pairs: 8.5e-8 of the result at k 272 (one chain of accumulations 1.6e-7, the kernel
+// above 8.8e-8). Rows
+// and columns past the end reread the last ones and are not stored. Bound by the outputs' bytes and the launch where it is used.
+__global__ __launch_bounds__(256) void mmf16_tile_kernel(const uint16_t* __restrict__ w, const float* __restrict__ x,
+                                                         float* __restrict__ y, int rows, int k, int ncols) {
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, kg = lane >> 4;
+    const int row0 = blockIdx.x * 64 + (wave & 1) * 32, col0 = blockIdx.y * 64 + (wave >> 1) * 32;
+    if (row0 >= rows || col0 >= ncols) return;
+    const uint16_t* wr[2];
+    const float* xr[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        wr[i] = w + (size_t)min(row0 + 16 * i + r, rows - 1) * k;
+        xr[i] = x + (size_t)min(col0 + 16 * i + r, ncols - 1) * k;
+    }
+    f32x4 sum[2][2] = {};
+    struct Step {
+        h8 a[2];
+        float4 xv[2][2];
+        __device__ void load(const uint16_t* const (&wr)[2], const float* const (&xr)[2], int at) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                a[i] = *reinterpret_cast<const h8*>(wr[i] + at);
+                const float4* xp = reinterpret_cast<const float4*>(xr[i] + at);
+                xv[i][0] = xp[0];
+                xv[i][1] = xp[1];
+            }
+        }
+    };
+    auto product = [&](const Step& st, bool in, f32x4 (&to)[2][2]) {  // to += (in: this lane's values are in the row)
+        const h8 zero = {};
+        h8 a[2], hi[2], lo[2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            splitHiLo(st.xv[i][0], st.xv[i][1], hi[i], lo[i]);
+            a[i] = in ? st.a[i] : zero;
+            hi[i] = in ? hi[i] : zero;
+            lo[i] = in ? lo[i] : zero;
+        }
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                f32x4 p = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[t], lo[c], f32x4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+                to[t][c] += __builtin_amdgcn_mfma_f32_16x16x32_f16(a[t], hi[c], p, 0, 0, 0);
+            }
+    };
+    int k0 = 8 * kg;
+    Step st[2];
+    for (; k0 - 8 * kg + 64 <= k; k0 += 64) {  // two steps' loads together
+        st[0].load(wr, xr, k0);
+        st[1].load(wr, xr, k0 + 32);
+        f32x4 two[2][2] = {};
+        product(st[0], true, two);
+        product(st[1], true, two);
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int c = 0; c < 2; ++c) sum[t][c] += two[t][c];
+    }
+    for (; k0 - 8 * kg < k; k0 += 32) {  // (past the row: its first values, unused)
+        const bool in = k0 < k;
+        st[0].load(wr, xr, in ? k0 : 0);
+        product(st[0], in, sum);
+    }
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            const int row = row0 + 16 * t + 4 * kg, col = col0 + 16 * c + r;
+            if (row < rows && col < ncols) *reinterpret_cast<f32x4u*>(y + (size_t)col * rows + row) = sum[t][c];  // rows % 8 == 0
+        }
+}
+
 // ---- any even k: one thread per (row, column), the reference's loop (llm_reference.cpp:756-764).
 __global__ __launch_bounds__(256) void mmf16_simple_kernel(const uint32_t* __restrict__ w, const float* __restrict__ x,
                                                            float* __restrict__ y, int rows, int k, int ncols) {
@@ -286,11 +364,25 @@ int launchMatmulF16(const void* w, const float* x, float* y, int rows, int k, in
             if (int e = launchMatmulF16(w, x + (size_t)c0 * k, y + (size_t)c0 * rows, rows, k, std::min(kMaxCols, ncols - c0), s))
                 return e;
     } else if (a16 && k % 16 == 0) {
-        // the smallest tile whose workgroups run at once on the 256 CUs (a second round costs more than a larger
+        const auto wgs = [&](int t, int c) { return (long long)((rows + 16 * t - 1) / (16 * t)) * ((ncols + 16 * c - 1) / (16 * c)); };
+        const long long cus = cuCount(), n42 = wgs(4, 2);
+        // Rows much shorter than the chunk of 256 values leave most of the K split's wavefronts without work, and each
+        // workgroup pays for all of them: once per round of workgroups over the GPU (us, K split / tile per wavefront: 4096 rows x
+        // 2048 columns, k 64 58.9 / 27.9, 128 58.8 / 36.8; 512 columns, k 128 24.6 / 19.3, 272 28.0 / 21.2; 20480 rows, 12 columns,
+        // k 288 19.4 / 17.4), little within one round (16384 rows, 9 columns, k 16: 14.6 / 13.1),
+        // nothing where that is not half full (64 rows, 512 columns, k 16: 13.6 / 14.4).
+        const bool tile = n42 < cus / 2 ? false
+                          : n42 <= cus  ? k <= (ncols <= 16 ? 128 : 64)
+                                        : k < 192 || (k < 352 && (k % 32 || (ncols <= 40 && n42 <= 2 * cus)));
+        if (tile) {
+            hipLaunchKernelGGL(mmf16_tile_kernel, dim3((rows + 63) / 64, (ncols + 63) / 64), dim3(256), 0, s, wh, x, y, rows,
+                               k, ncols);
+            return fromHip(hipGetLastError(), "matmul_f16");
+        }
+        // the smallest tile whose workgroups run at once on the CUs (a second round costs more than a larger
         // tile: 1024 x 4096, 77 columns 12.4 us on 16 x 16 (320 workgroups), 9.9 us on 32 x 16 (160), 11.3 us on
         // 64 x 16 (80)), else the largest (512 columns: 18.7 us on 64 x 32, 22.5 us on 64 x 16); three stages where they
         // fit
-        const auto wgs = [&](int t, int c) { return (long long)((rows + 16 * t - 1) / (16 * t)) * ((ncols + 16 * c - 1) / (16 * c)); };
         const dim3 block(64 * kF16Waves);
 #define KC_F16(TT, CC, SS)                                                                                             \
     {                                                                                                                  \
@@ -302,9 +394,9 @@ int launchMatmulF16(const void* w, const float* x, float* y, int rows, int k, in
         hipLaunchKernelGGL((mmf16_mfma_kernel<TT, CC, SS>), dim3((rows + 16 * TT - 1) / (16 * TT),                     \
                            (ncols + 16 * CC - 1) / (16 * CC)), block, lds, s, wh, x, y, rows, k, ncols);               \
     }
-        if (wgs(1, 1) <= 256) KC_F16(1, 1, 3)
-        else if (wgs(2, 1) <= 256) KC_F16(2, 1, 3)
-        else if (wgs(4, 1) <= 256) KC_F16(4, 1, 3)
+        if (wgs(1, 1) <= cus) KC_F16(1, 1, 3)
+        else if (wgs(2, 1) <= cus) KC_F16(2, 1, 3)
+        else if (wgs(4, 1) <= cus) KC_F16(4, 1, 3)
         else KC_F16(4, 2, 2)
 #undef KC_F16
     } else {

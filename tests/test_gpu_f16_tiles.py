@@ -22,6 +22,7 @@ def runtime():
     (8, 16, 9), (24, 240, 17), (40, 256, 16), (72, 272, 31), (520, 1040, 33),          # 16 x 16 tiles
     (1016, 512, 77), (1016, 768, 200), (2056, 272, 130), (4104, 528, 261),              # 32 x 16, 64 x 16, 64 x 32
     (8, 16, (1 << 20) + 20),                                                           # two launches
+    (16384, 16, 10), (4104, 144, 261), (2056, 176, 1030), (16392, 272, 40),             # a 32 x 32 tile per wavefront
 ])
 def test_matmul_f16_tiles(rows, k, ncols):
     print(f"matmul_f16 {rows} x {k} x {ncols}", flush=True)

@@ -131,3 +131,12 @@ def test_f16_limits(routes):
     names = [[g[0].split(",")[0] for g in c] for c in got]
     assert names == [["mmf16_mfma_kernel"], ["mmf16_mfma_kernel", "mmf16_vec_kernel"], ["mmf16_mfma_kernel"] * 3,
                      ["mmf16_mfma_kernel"], ["mmf16_vec_kernel"] * 2]
+
+
+def test_f16_short_rows(routes):
+    """Rows short of a K-split chunk, where the workgroups take several rounds: the kernel of one tile per wavefront."""
+    tile = [(4096, 128, 512), (4096, 144, 2048), (16384, 16, 9), (16384, 128, 16), (4096, 272, 512), (16384, 176, 1000),
+            (20480, 288, 12)]
+    split = [(64, 16, 512), (4096, 192, 512), (4096, 96, 64), (4096, 288, 512), (4096, 384, 512), (16384, 256, 1000)]
+    got = routes([("f16", c) for c in tile + split])
+    assert [g[0][0].split(",")[0] for g in got] == ["mmf16_tile_kernel"] * len(tile) + ["mmf16_mfma_kernel"] * len(split)
