@@ -1230,8 +1230,14 @@ size_t stagedActBytes(const kcMatmulKQ8Args& a) { return (actBytes(a.ncols, a.k)
 size_t stagedBytes(const kcMatmulKQ8Args& a, int ks) {
     return stagedActBytes(a) + (ks == 2 ? (size_t)a.rows * a.ncols * 4 : 0);
 }
+// Whether a by-name batch runs on the int8 kernel: of the staging it needs the partial sums alone.
+bool i8Batch(bool q6k, const kcMatmulKQ8Args& a) {
+    const MmPart part{a.qw, {a.y, nullptr}, a.rows, q6k ? 1 : 0};
+    return i8Group(&part, 1, a.xq, a.k / 256);
+}
 int runStaged(bool q6k, const kcMatmulKQ8Args& a, int ks, void* buf, hipStream_t s) {
-    float* partial = ks == 2 ? reinterpret_cast<float*>(static_cast<char*>(buf) + stagedActBytes(a)) : nullptr;
+    float* partial = nullptr;
+    if (ks == 2) partial = reinterpret_cast<float*>(static_cast<char*>(buf) + (i8Batch(q6k, a) ? 0 : stagedActBytes(a)));
     const MmPart part{a.qw, {a.y, partial}, a.rows, q6k ? 1 : 0};
     if (int st = runMfmaH(&part, 1, a.xq, a.k, a.ncols, ks, buf, s)) return st;
     if (ks == 1) return 0;
@@ -1337,6 +1343,10 @@ int launchMatmulMfma(bool q6k, const kcMatmulKQ8Args& a, hipStream_t s) {
     // fp16 activations staged by direct loads (a per-stream buffer, addressed with 32-bit offsets)
     if (path != 5 && (size_t)a.ncols * a.k * 2 < (1ull << 32)) {
         const int ks = stagedKs(q6k, a);
+        if (i8Batch(q6k, a)) {  // no fp16 activations; without the partial sums' buffer one K range
+            void* buf = ks == 2 ? streamScratch(s, (size_t)a.rows * a.ncols * 4) : nullptr;
+            return runStaged(q6k, a, buf ? 2 : 1, buf, s);
+        }
         if (void* buf = streamScratch(s, stagedBytes(a, ks))) return runStaged(q6k, a, ks, buf, s);
     }
     return q6k ? runMfma8<true, 1>(a, s) : runMfma8<false, 1>(a, s);

@@ -29,9 +29,11 @@ def launched(f):
     return out
 
 
-def matmul(qtype, rows, k, ncols):
+def matmul(qtype, rows, k, ncols, no_scratch=0):
     w, x, y = (kc.Buffer(n) for n in (kc.stream_bytes(qtype, rows, k), k // 256 * 340 * ncols, 4 * rows * ncols))
+    stub.stub_capturing(no_scratch)
     r = launched(lambda: kc.launch("matmul_%s_q8kx8" % qtype, kc.MatmulKQ8Args(w.ptr, x.ptr, y.ptr, None, rows, k, ncols, 8)))
+    stub.stub_capturing(0)
     for b in (w, x, y):
         b.free()
     return r
@@ -117,7 +119,7 @@ def test_unstaged_batches_keep_the_prefill_kernel(routes):
     """64 columns and more that cannot be staged run on the prefill kernel that stages nothing, not on the short-batch one:
     past the fp16 layout's 32-bit offsets (a down projection of 16384 columns of 131072 values), and with no staging buffer."""
     down, groups = routes([("model", [16384], dict(types={"w_down": "q4k"}, n_embd=256, n_head=2, n_head_kv=2, n_ff=131072)),
-                           ("model", [80], dict(types={"w_down": "q4k"}, options={"prefill_act": 1}, no_scratch=1))])
+                           ("model", [80], dict(types={"w_down": "q4k"}, n_embd=512, n_head=4, options={"prefill_act": 1}, no_scratch=1))])
     for got, count in ((down, 1), (groups, 2 * 4 + 2 + 1)):  # (q / k / v and o of two layers, gate / up and down of one)
         names = [g[0].split(",")[0] for g in got if g[0].startswith("matmul_")]
         assert "matmul_short_kernel" not in names and names.count("matmul_kq_mfma8_kernel") == count, names
@@ -140,3 +142,12 @@ def test_f16_short_rows(routes):
     split = [(64, 16, 512), (4096, 192, 512), (4096, 96, 64), (4096, 288, 512), (4096, 384, 512), (16384, 256, 1000)]
     got = routes([("f16", c) for c in tile + split])
     assert [g[0][0].split(",")[0] for g in got] == ["mmf16_tile_kernel"] * len(tile) + ["mmf16_mfma_kernel"] * len(split)
+
+
+def test_int8_prefill_without_staging(routes):
+    """A Q6_K batch on the int8 kernel stages no activations: with no staging buffer it keeps that kernel, in one K range."""
+    got = routes([("matmul", ("q6k", 16384, 3072, 128), dict(no_scratch=1))]
+                 + [("matmul", ("q6k", 1024, 3072, 128), dict(no_scratch=n)) for n in (1, 0)])
+    assert [[g[0].split(",")[0] for g in c] for c in got] == [["matmul_i8_kernel"], ["matmul_i8_kernel"],
+                                                              ["matmul_i8_kernel", "add_partial_kernel"]]
+    assert [c[0][3] for c in got] == [1, 1, 2]
