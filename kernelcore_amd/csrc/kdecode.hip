@@ -1478,8 +1478,9 @@ int launchDecodeMatvec(int pro, int epi, DmvArgs a, hipStream_t s) {
     const dim3 grid(wgs), block(64 * nw);
 #define KC_DMV(P, Q, N8) \
     if (pro == P && epi == Q && n8 == N8) hipLaunchKernelGGL((dmv_kernel<P, Q, N8>), grid, block, lds, s, a);
-    // The slabs issued before and during the norm prologue (8 lanes per block): see the kernel. Option
-    // "swiglu_pre": 1-13 that many before in the SwiGLU workgroups (in steps of three), 14 none.
+    // The slabs issued before and during the norm prologue (8 lanes per block): see the kernel. The counts are measured on
+    // rows of 3072 (12 wavefronts per CU), not derived from a shape's wavefronts per CU. Option "swiglu_pre": slabs before in
+    // the SwiGLU workgroups, 1-3 three, 4-6 six, 7-13 nine, 14 none.
     const int po = option("swiglu_pre");
     if (pro == kProNorm && epi == kEpiSwiglu && n8) {
         if (po == 0) hipLaunchKernelGGL((dmv_kernel<kProNorm, kEpiSwiglu, true, 3, 3>), grid, block, lds, s, a);

@@ -1322,7 +1322,9 @@ int launchMatmulKqNoAlloc(bool q6k, bool per256, const kcMatmulKQ8Args& a, hipSt
 // K split in two where one K range leaves compute units idle. The producer-wavefront kernel holds
 // one workgroup per CU, so it splits only when twice its workgroups still run at once (a 4096-row
 // matrix over 1024 columns, 256 workgroups: 45.7 us in one K range, 51.5 us in two, the partial
-// sums' extra pass included); the other kernels split below two 128-row workgroups per CU.
+// sums' extra pass included); the other kernels split below two 128-row workgroups per CU. The int8
+// kernel takes the producer-wavefront kernel's rule, which is not made from its own tiles (128 rows, 64 or
+// 128 columns, two workgroups per CU).
 int matmulKs(int rows, int k, int ncols, bool q6) {
     if (k / 256 < 2) return 1;
     const long long ct = (ncols + 63) / 64;

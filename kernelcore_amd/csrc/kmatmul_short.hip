@@ -13,7 +13,8 @@
 // applied to the op's 4 sums per lane by a 24-bit multiply-add: 4 vector ops per op, whatever the scale,
 // where scaling the weights before the op would need two ops per sub-block (6-bit scale times 4-bit
 // value does not fit a byte). Q6_K's scales cover 16 values: each op takes half of its lanes' values
-// (the other half zeroed), two ops per 32 values.
+// (the other half zeroed), two ops per 32 values -- as many as the scaled weights in two bytes would take
+// (kmatmul_i8.hip), a form not measured here.
 //
 // Measured (this kernel alone, against the column-tiled kernel): 8192 x 3072 Q4_K, 12 columns 23.0 -> 7.5 us,
 // 37 columns 46.9 -> 12.4 us, 63 columns 68.7 -> 18.5 us; 3072 x 8192 Q6_K, 2 columns 21.2 -> 9.9 us, 12 columns
