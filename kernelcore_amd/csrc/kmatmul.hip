@@ -185,6 +185,10 @@ int launchMatmulFew(bool q6k, bool per256, const kcMatmulKQ8Args& a, hipStream_t
     return launchMatmulCols(q6k, per256, a, s);
 }
 
+// The line at 64 columns is one for all sizes, and not the better one everywhere (us by name, short batch at 63 columns / prefill
+// kernel at 64): Q4_K 1024 x 3072 22.3 / 28.6, 3072 x 8192 32.3 / 48.1, 4096 x 12288 44.1 / 64.5, 8192 x 3072 27.7 / 30.4, but
+// 14336 x 4096 44.7 / 35.4 and 16384 x 3072 42.7 / 32.1 (40 columns 31.6 / 30.7); Q6_K 1024 x 3072 23.3 / 27.3, 3072 x 8192
+// 34.5 / 44.4, 8192 x 3072 29.2 / 29.0, 14336 x 4096 47.8 / 33.9, 128256 x 2048 175 / 84.
 int launchMatmulKq(bool q6k, bool per256, const kcMatmulKQ8Args& a, hipStream_t s) {
     // "matmul_path": 0 default (per-256 slots: the short-batch kernel, the
     // prefill MFMA kernel from 64 columns), 1 column tiles; 2 and up

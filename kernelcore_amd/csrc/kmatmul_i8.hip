@@ -13,9 +13,11 @@
 // poorly at two wavefronts per SIMD (timing copies, 8192 x 6144 x 512, 82 us: 50 without unpacking, 37 with matrix ops
 // and barriers alone). Hence a workgroup of four wavefronts x 32 rows and 64 or 128 columns, two per CU, each wavefront
 // unpacking its rows' weights once into registers for all its column blocks, and a block's combine issued between the
-// next block's matrix ops. Measured against the fp16 producer-wavefront kernel (us): 512 columns, k 3072: 8192 rows 51.9 ->
-// 44.0, 2048 rows 32.6 -> 21.4, 16384 rows 95.1 -> 65.6; 3072 x 8192: 64 columns 56.2 -> 33.7, 200 57.7 -> 35.2, 700 104.5 ->
-// 91.5, 2048 204 -> 135; 14336 x 4096, 65 columns 36.2 -> 32.3; 128 x 3072 25.9 -> 16.2: faster at every size measured.
+// next block's matrix ops. Measured against the fp16 producer-wavefront kernel (us, kernel times of one trace, without that
+// kernel's conversion launch of 5): 512 columns, k 3072: 8192 rows 54.0 -> 47.1, 2048 rows 26.1 -> 20.8, 16384 rows 105 -> 71.4;
+// 3072 x 8192: 64 columns 51.0 -> 31.7, 200 56.4 -> 35.8, 700 110 -> 102, 2048 231 -> 161; 14336 x 4096, 65 columns 34.0 -> 30.0;
+// 128 x 3072, 512 columns 22.6 -> 15.6; 24576 x 4096, 1024 columns 380 -> 257. Faster at all of 181 sizes, 0.73 of the time
+// (geometric mean).
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -301,8 +303,9 @@ int launchMatmulI8(MfmaGroup g, const int* xq, int nsb, int ncols, hipStream_t s
         tiles += (g.p[i].rows + kRows - 1) / kRows;
     }
     // 128 columns per workgroup unpack each weight half as often, but pay only where two such workgroups per CU
-    // have work (k 3072, 512 columns: 16384 rows 58.4 us against 79 with 64; 8192 rows 45 against 39) and more than 64
-    // columns (64 columns, half a tile of padding: 128256 x 3072 134 us against 111)
+    // have work (kernel times of one trace, k 3072, 512 columns: 16384 rows 71.4 us against 110 with 64; 2048 rows 25.3 against
+    // 20.8; 8192 rows 47 either way) and more than 64 columns (64 columns, half a tile of padding: 128256 x 3072 127 us
+    // against 112)
     const long long wgs = (long long)tiles * ((ncols + 127) / 128) * g.ks;
     return ncols > 64 && wgs >= 2LL * cuCount() ? launch<4>(g, tiles, xq, nsb, ncols, s) : launch<2>(g, tiles, xq, nsb, ncols, s);
 }

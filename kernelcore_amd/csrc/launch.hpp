@@ -40,7 +40,7 @@ int launchMatvecKq(bool q6k, const kcMatvecQ4Q8Args& a, hipStream_t s);
 // kmatmul.hip: column-tiled matmul (any ncols; bit-identical per column to the reference).
 int launchMatmulCols(bool q6k, bool per256, const kcMatmulKQ8Args& a, hipStream_t s);
 // The batches the prefill MFMA kernel does not take: per-256 slots on the short-batch kernel
-// (kmatmul_short.hip), else column tiles.
+// (kmatmul_short.hip) but for two or three columns of a tall matrix, else column tiles.
 int launchMatmulFew(bool q6k, bool per256, const kcMatmulKQ8Args& a, hipStream_t s);
 // kmatmul_mfma.hip: K-quant x per-256 activations on MFMA (large batches).
 int launchMatmulMfma(bool q6k, const kcMatmulKQ8Args& a, hipStream_t s);
